@@ -135,6 +135,7 @@ uint64_t Engine::submit(std::shared_ptr<const RunHost> h, uint64_t id) {
     r->hp = std::move(h);
     r->footprint = footprint_bytes(*r->hp);
     r->st = st_;
+    r->stage = ctx_->stage;
     r->t_submit = Clock::now();
     pending_.push_back(r);
     return id;
@@ -1295,54 +1296,34 @@ void Engine::sample_frontier(const std::vector<SampledKids>& kids, uint32_t nC, 
 // result readback
 // ------------------------------------------------------------------------------------------
 
-struct RunTables {
-    std::vector<uint64_t> hash;
-    std::vector<uint32_t> step, creator;
-    std::vector<uint32_t> ev_in, ev_rule, ev_step;
-    std::vector<uint64_t> ev_prod, ev_tr;
+// The event tables the causal triples are derived from (the other arrays: hgx_readback.hip), in
+// event order, and the generation of every state. Segments lie in state-id order, so each one's
+// part is copied in place.
+struct EventTables {
+    std::vector<uint32_t> in, rule, step;          // step: of every state
+    std::vector<uint64_t> tr;
 };
 
-static RunTables run_tables(const RunRec& R) {
-    RunTables T;
-    const uint64_t ns = R.states;
-    const uint32_t nroots = R.hp->n_roots();
+static EventTables event_tables(const RunRec& R) {
+    EventTables T;
+    const uint64_t ns = R.states, nroots = R.hp->n_roots();
     const uint64_t ne = ns >= nroots ? ns - nroots : 0;
-    T.hash.resize(ns); T.step.resize(ns); T.creator.assign(ns, 0xFFFFFFFFu);
-    T.ev_in.resize(ne); T.ev_rule.resize(ne); T.ev_step.resize(ne); T.ev_prod.resize(ne); T.ev_tr.resize(ne);
+    T.step.resize(ns); T.in.resize(ne); T.rule.resize(ne); T.tr.resize(ne);
+    uint64_t s = 0;
     for (size_t k = 0; k < R.segs.size(); ++k) {
         const Segment& sg = R.segs[k];
         const uint32_t m = sg.e - sg.b;
-        if (!m) continue;
-        std::vector<uint64_t> h(m);
-        std::vector<uint32_t> sid(m);
-        std::vector<uint8_t> dep(m);
-        d2h(h.data(), sg.g->v.hash + sg.b, m, R.st);
-        d2h(sid.data(), sg.g->v.sid + sg.b, m, R.st);
-        d2h(dep.data(), sg.g->v.depth + sg.b, m, R.st);
-        std::vector<uint32_t> in, rule;
-        std::vector<uint64_t> prod, tr;
-        const bool events = k > 0;                  // the first segment holds the roots
-        if (events) {
-            in.resize(m); rule.resize(m); prod.resize(m); tr.resize(m);
-            d2h(in.data(), sg.g->ev.in_state + sg.b, m, R.st);
-            d2h(rule.data(), sg.g->ev.rule + sg.b, m, R.st);
-            d2h(prod.data(), sg.g->ev.prod + sg.b, m, R.st);
-            d2h(tr.data(), sg.g->ev.tr + sg.b, m, R.st);
+        if (s + m > ns) throw Error{HGX_ERR_DEVICE, "state id out of range in readback"};
+        std::fill(T.step.begin() + s, T.step.begin() + s + m, (uint32_t)k);
+        if (k > 0) {                                // the first segment holds the roots
+            const uint64_t e = s - nroots;
+            d2h(T.in.data() + e, sg.g->ev.in_state + sg.b, m, R.st);
+            d2h(T.rule.data() + e, sg.g->ev.rule + sg.b, m, R.st);
+            d2h(T.tr.data() + e, sg.g->ev.tr + sg.b, m, R.st);
         }
-        HIP_TRY(hipStreamSynchronize(R.st));
-        for (uint32_t i = 0; i < m; ++i) {
-            const uint32_t s = sid[i];
-            if (s >= ns) throw Error{HGX_ERR_DEVICE, "state id out of range in readback"};
-            T.hash[s] = h[i];
-            T.step[s] = dep[i];
-            if (events) {
-                const uint32_t e = s - nroots;
-                T.creator[s] = e;
-                T.ev_in[e] = in[i]; T.ev_rule[e] = rule[i]; T.ev_step[e] = dep[i];
-                T.ev_prod[e] = prod[i]; T.ev_tr[e] = tr[i];
-            }
-        }
+        s += m;
     }
+    HIP_TRY(hipStreamSynchronize(R.st));
     return T;
 }
 
@@ -1735,59 +1716,6 @@ extern "C" void hgx_result_release_many(hgx_result* const* rs, uint32_t n) {
     for (uint32_t i = 0; i < n; ++i) delete rs[i];
 }
 
-extern "C" int hgx_result_states(const hgx_result* r, uint64_t* hash, uint32_t* step, uint32_t* creator,
-                                 uint64_t cap) {
-    if (!r || cap < r->run->counts.raw_states) return HGX_ERR_INVALID;
-    try {
-        RunTables T = run_tables(*r->run);
-        for (uint64_t s = 0; s < r->run->states; ++s) {
-            if (hash) hash[s] = T.hash[s];
-            if (step) step[s] = T.step[s];
-            if (creator) creator[s] = T.creator[s];
-        }
-        return HGX_OK;
-    } catch (const Error& e) {
-        return e.code;
-    }
-}
-
-extern "C" int hgx_result_events(const hgx_result* r, hgx_event* out, uint64_t cap) {
-    if (!r || (!out && r->run->events) || cap < r->run->events) return HGX_ERR_INVALID;
-    try {
-        RunTables T = run_tables(*r->run);
-        const uint32_t nroots = r->run->hp->n_roots();
-        for (uint64_t e = 0; e < r->run->events; ++e)
-            out[e] = hgx_event{T.ev_in[e], (uint32_t)(e + nroots), T.ev_rule[e], T.ev_step[e]};
-        return HGX_OK;
-    } catch (const Error& e) {
-        return e.code;
-    }
-}
-
-extern "C" int hgx_result_causal(const hgx_result* r, hgx_pair* pairs, uint8_t* in_tr, uint64_t cap) {
-    if (!r) return HGX_ERR_INVALID;
-    const RunRec& R = *r->run;
-    if (!(R.hp->flags & HGX_REC_CAUSAL) || cap < R.counts.causal_pairs) return HGX_ERR_INVALID;
-    try {
-        RunTables T = run_tables(R);
-        uint64_t o = 0;
-        for (uint64_t c = 0; c < R.events; ++c) {
-            for (uint64_t m = T.ev_prod[c]; m; m &= m - 1) {
-                const uint32_t s = (uint32_t)__builtin_ctzll(m);
-                uint32_t x = T.ev_in[c];                 // walk up the lineage to generation s
-                while (T.step[x] > s) x = T.ev_in[T.creator[x]];
-                if (o >= cap) return HGX_ERR_INVALID;
-                if (pairs) pairs[o] = hgx_pair{T.creator[x], (uint32_t)c};
-                if (in_tr) in_tr[o] = (uint8_t)((T.ev_tr[c] >> s) & 1u);
-                ++o;
-            }
-        }
-        return HGX_OK;
-    } catch (const Error& e) {
-        return e.code;
-    }
-}
-
 extern "C" int hgx_result_causal_triples(const hgx_result* r, hgx_triple* triples, uint8_t* in_tr, uint64_t cap) {
     if (!r) return HGX_ERR_INVALID;
     const RunRec& R = *r->run;
@@ -1795,11 +1723,12 @@ extern "C" int hgx_result_causal_triples(const hgx_result* r, hgx_triple* triple
         cap < R.counts.causal_triples)
         return HGX_ERR_INVALID;
     try {
-        RunTables T = run_tables(R);
+        EventTables T = event_tables(R);
         const uint32_t nroots = R.hp->n_roots();
         // producer generation of every consumed edge, per event
         std::vector<uint8_t> cps;
         uint32_t K = 0;
+        uint64_t e0 = 0;                                       // events before the segment
         for (size_t k = 1; k < R.segs.size(); ++k) {          // segment 0 holds the roots
             const Segment& sg = R.segs[k];
             const uint32_t m = sg.e - sg.b;
@@ -1808,54 +1737,28 @@ extern "C" int hgx_result_causal_triples(const hgx_result* r, hgx_triple* triple
             const uint32_t gk = sg.g->ev.cK;
             if (!K) { K = 16; cps.assign((size_t)R.events * K, 0); }
             std::vector<uint8_t> rows((size_t)m * gk);
-            std::vector<uint32_t> sid(m);
             d2h(rows.data(), sg.g->ev.cps + (size_t)sg.b * gk, rows.size(), R.st);
-            d2h(sid.data(), sg.g->v.sid + sg.b, m, R.st);
             HIP_TRY(hipStreamSynchronize(R.st));
-            for (uint32_t i = 0; i < m; ++i) {
-                const uint64_t e = (uint64_t)sid[i] - nroots;
-                if (e >= R.events) throw Error{HGX_ERR_DEVICE, "event id out of range in readback"};
-                std::memcpy(&cps[e * K], &rows[(size_t)i * gk], std::min<uint32_t>(gk, K));
-            }
+            if (e0 + m > R.events) throw Error{HGX_ERR_DEVICE, "event id out of range in readback"};
+            for (uint32_t i = 0; i < m; ++i)
+                std::memcpy(&cps[(e0 + i) * K], &rows[(size_t)i * gk], std::min<uint32_t>(gk, K));
+            e0 += m;
         }
         uint64_t o = 0;
         for (uint64_t c = 0; c < R.events; ++c) {
-            const uint32_t nl = R.hp->rules.at(T.ev_rule[c]).n_lhs;
+            const uint32_t nl = R.hp->rules.at(T.rule[c]).n_lhs;
             for (uint32_t t = 0; t < nl; ++t) {
                 const uint32_t ps = cps[c * K + t];
                 if (!ps) continue;
-                uint32_t x = T.ev_in[c];                 // up the lineage to generation ps
-                while (T.step[x] > ps) x = T.ev_in[T.creator[x]];
+                uint32_t x = T.in[c];                 // up the lineage to generation ps
+                while (T.step[x] > ps) x = T.in[x - nroots];
                 if (o >= cap) return HGX_ERR_INVALID;
-                if (triples) triples[o] = hgx_triple{T.creator[x], (uint32_t)c, t};
-                if (in_tr) in_tr[o] = (uint8_t)((T.ev_tr[c] >> ps) & 1u);
+                if (triples) triples[o] = hgx_triple{x - nroots, (uint32_t)c, t};
+                if (in_tr) in_tr[o] = (uint8_t)((T.tr[c] >> ps) & 1u);
                 ++o;
             }
         }
         return o == R.counts.causal_triples ? HGX_OK : HGX_ERR_DEVICE;
-    } catch (const Error& e) {
-        return e.code;
-    }
-}
-
-extern "C" int hgx_result_branchial(const hgx_result* r, hgx_pair* pairs, uint64_t cap) {
-    if (!r) return HGX_ERR_INVALID;
-    const RunRec& R = *r->run;
-    if (!(R.hp->flags & HGX_REC_BRANCHIAL) || !(R.hp->flags & HGX_REC_RELATIONS)) return HGX_ERR_INVALID;
-    if (cap < R.counts.branchial_pairs) return HGX_ERR_INVALID;
-    try {
-        uint64_t o = 0;
-        for (const Segment& sg : R.segs) {
-            if (sg.br_e <= sg.br_b || !sg.g->br_pairs) continue;
-            std::vector<uint32_t> tmp(2 * (sg.br_e - sg.br_b));
-            d2h(tmp.data(), sg.g->br_pairs + 2 * sg.br_b, tmp.size(), R.st);
-            HIP_TRY(hipStreamSynchronize(R.st));
-            for (uint64_t i = 0; i < sg.br_e - sg.br_b; ++i) {
-                if (o >= cap) return HGX_ERR_INVALID;
-                pairs[o++] = hgx_pair{tmp[2 * i], tmp[2 * i + 1]};
-            }
-        }
-        return HGX_OK;
     } catch (const Error& e) {
         return e.code;
     }

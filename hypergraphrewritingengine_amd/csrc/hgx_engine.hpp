@@ -75,6 +75,7 @@ struct RunRec {
     std::unordered_set<uint64_t> q_seen;
     hgx_counts counts{};
     hipStream_t st = nullptr;        // the context's stream (contexts outlive results)
+    std::shared_ptr<PinnedStage> stage;    // the context's readback buffers
     Clock::time_point t_submit, t_admit, t_done;
     double device_ms = 0;
 };

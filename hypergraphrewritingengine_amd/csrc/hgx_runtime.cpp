@@ -80,6 +80,46 @@ std::vector<Chunk> ChunkPool::take_held() {
     return h;
 }
 
+void PinnedStage::destroy(Buf& b) {
+    for (hipEvent_t e : b.ev)
+        if (e) (void)hipEventDestroy(e);
+    if (b.p) (void)hipHostFree(b.p);
+    b = Buf{};
+}
+
+PinnedStage::~PinnedStage() {
+    for (auto& b : idle_) destroy(b);
+}
+
+StageLease::StageLease(PinnedStage& s) : s_(s) {
+    {
+        std::lock_guard<std::mutex> g(s_.mu_);
+        if (!s_.idle_.empty()) {
+            b_ = s_.idle_.back();
+            s_.idle_.pop_back();
+            return;
+        }
+    }
+    try {
+        HIP_TRY(hipHostMalloc((void**)&b_.p, 2 * kHalf, hipHostMallocDefault));
+        for (hipEvent_t& e : b_.ev) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    } catch (...) {
+        PinnedStage::destroy(b_);
+        throw;
+    }
+}
+
+StageLease::~StageLease() {
+    {
+        std::lock_guard<std::mutex> g(s_.mu_);
+        if (s_.idle_.size() < PinnedStage::kKeep) {
+            s_.idle_.push_back(b_);
+            return;
+        }
+    }
+    PinnedStage::destroy(b_);
+}
+
 Arena::~Arena() { release(); }
 
 void Arena::release() {
@@ -526,6 +566,7 @@ extern "C" int hgx_ctx_create(int device, uint64_t budget_bytes, hgx_ctx** out) 
     (void)hipMemGetInfo(&freeb, &totalb);
     const uint64_t budget = budget_bytes ? budget_bytes : (uint64_t)(freeb * 0.8);
     c->pool = std::make_shared<ChunkPool>(budget, (size_t)64 << 20);
+    c->stage = std::make_shared<PinnedStage>(device);
     c->num_cu = (uint32_t)prop.multiProcessorCount;
     c->max_lds = (uint32_t)prop.sharedMemPerBlock;
     (void)tune_load(c, default_tune_cache());   // tuned launch shapes of this device, when cached

@@ -98,6 +98,44 @@ private:
     size_t slab_used_ = 0;
 };
 
+// Pinned host buffers that results are read back through, one lease per call in flight (results
+// may be read by several threads). At most kKeep idle buffers are kept; a lease beyond them
+// allocates one and frees it. Owned by the context and by every run that may be read.
+class PinnedStage {
+public:
+    explicit PinnedStage(int device) : device_(device) {}
+    ~PinnedStage();
+    PinnedStage(const PinnedStage&) = delete;
+    PinnedStage& operator=(const PinnedStage&) = delete;
+    int device() const { return device_; }
+
+private:
+    friend class StageLease;
+    struct Buf {
+        uint8_t* p = nullptr;
+        hipEvent_t ev[2] = {nullptr, nullptr};
+    };
+    static constexpr size_t kKeep = 4;
+    static void destroy(Buf& b);
+    int device_;
+    std::mutex mu_;
+    std::vector<Buf> idle_;
+};
+class StageLease {
+public:
+    static constexpr size_t kHalf = (size_t)2 << 20;
+    explicit StageLease(PinnedStage& s);
+    ~StageLease();
+    StageLease(const StageLease&) = delete;
+    StageLease& operator=(const StageLease&) = delete;
+    uint8_t* half(uint64_t k) const { return b_.p + k * kHalf; }
+    hipEvent_t event(uint64_t k) const { return b_.ev[k]; }
+
+private:
+    PinnedStage& s_;
+    PinnedStage::Buf b_;
+};
+
 template <class T>
 T* dalloc(Arena& a, size_t n) { return (T*)a.alloc(sizeof(T) * (n ? n : 1)); }
 
@@ -258,6 +296,7 @@ struct hgx_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
     std::shared_ptr<hgx::ChunkPool> pool;
+    std::shared_ptr<hgx::PinnedStage> stage;     // pinned buffers of the result readbacks
     std::string err;
     std::string info;
     uint32_t num_cu = 256;
