@@ -161,6 +161,20 @@ __device__ inline uint32_t wave_incl_scan_u32(uint32_t v) {
     return v;
 }
 
+__device__ inline uint64_t wave_lane_u64(uint64_t v, uint32_t lane) {
+    const uint32_t lo = __shfl((uint32_t)v, (int)lane, WAVE), hi = __shfl((uint32_t)(v >> 32), (int)lane, WAVE);
+    return ((uint64_t)hi << 32) | lo;
+}
+
+__device__ inline uint64_t wave_incl_scan_u64(uint64_t v) {
+    const uint32_t l = lane_id();
+    for (int o = 1; o < WAVE; o <<= 1) {
+        const uint32_t lo = __shfl_up((uint32_t)v, o, WAVE), hi = __shfl_up((uint32_t)(v >> 32), o, WAVE);
+        if (l >= (uint32_t)o) v += ((uint64_t)hi << 32) | lo;
+    }
+    return v;
+}
+
 // Exclusive prefix sum of a[0..n) in LDS, in place, by one wave; returns the total.
 __device__ __forceinline__ uint32_t wave_excl_scan_lds(uint32_t* a, uint32_t n) {
     const uint32_t l = lane_id();

@@ -499,7 +499,7 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
             HIP_TRY(launch_fill(cnt, 0, sizeof(uint32_t) * (n + 1), st));
             launch_classes(false, mcls_count, "k_match_count", match_bytes + n * 4ull);
             scan_u32_to_u64(tmp, cnt, moff, n, st);
-            HIP_TRY(launch_run_totals(moff, ma.state_edges, cnt, F_->v.ne, d_sbeg_, d_send_, cap_slots_, d_tot_,
+            HIP_TRY(launch_run_totals(moff, ma.state_edges, cnt, F_->v.ne, F_->v.run, n, d_sbeg_, d_send_, d_tot_,
                                       d_run_edges_, d_run_pe_, st));
             // per-slot child edges, totals and parent edges are adjacent
             // ([edges cap][totals cap + 1][parent edges cap]): one read

@@ -1464,28 +1464,58 @@ hipError_t launch_copy_roots(const RootCopy* items, uint32_t n, const GenView& v
     return hipGetLastError();
 }
 
-// Per-run match totals of a generation: runs' states are contiguous ranges.
-// One wave per run: its matches from the offsets; its children's edges and the edges of its
-// states that have matches (the parents its expansion reads), summed over its states -- a
-// per-state store and these sums instead of every state adding to shared counters.
+// Per-run match totals of a generation: runs' states are contiguous ranges. For each run, its
+// children's edges and the edges of its states that have matches (the parents its expansion reads)
+// are summed into its slot (zero before the launch), its matches come from the offsets. A wave takes
+// kTotalsChunk consecutive states, 64 at a time: lanes of one run keep running sums that are
+// added once per chunk, and a group holding several runs is summed by segments with one scan, so
+// neither one run of 300 k states (one wave per run: 2.05 ms a pass, so 0.04) nor a generation of
+// one state per run (run after run in a chunk: 0.59 ms a batched pass, so 0.10) is left to one
+// wave's latency.
+constexpr uint32_t kTotalsChunk = 512;
+__device__ __forceinline__ void add_run_totals(uint64_t* edges, uint64_t* parent_edges, uint32_t r, uint64_t sum,
+                                               uint64_t pe) {
+    if (sum) atomicAdd((unsigned long long*)&edges[r], (unsigned long long)sum);
+    if (pe) atomicAdd((unsigned long long*)&parent_edges[r], (unsigned long long)pe);
+}
 __global__ void k_run_totals(const uint64_t* moff, const uint64_t* state_edges, const uint32_t* cnt,
-                             const uint32_t* ne, const uint32_t* run_sbeg, const uint32_t* run_send,
-                             uint32_t nruns, uint64_t* tot, uint64_t* edges, uint64_t* parent_edges) {
-    const uint32_t r = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE, l = lane_id();
-    if (r >= nruns) return;
-    const uint32_t b = run_sbeg[r], e = run_send[r];
-    uint64_t sum = 0, pe = 0;
-    for (uint32_t s = b + l; s < e; s += WAVE) {
-        sum += state_edges[s];
-        pe += cnt[s] ? ne[s] : 0u;
+                             const uint32_t* ne, const uint32_t* run, uint32_t n, const uint32_t* run_sbeg,
+                             const uint32_t* run_send, uint64_t* tot, uint64_t* edges, uint64_t* parent_edges) {
+    const uint32_t c = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE, l = lane_id();
+    const uint32_t first = c * kTotalsChunk, end = min(n, first + kTotalsChunk);
+    uint64_t sum = 0, pe = 0;                           // this lane's states of run `cur`
+    uint32_t cur = INV;
+    auto flush = [&] {
+        if (cur == INV) return;
+        const uint64_t a = wave_sum_u64(sum), b = wave_sum_u64(pe);
+        if (l == 0) add_run_totals(edges, parent_edges, cur, a, b);
+        sum = pe = 0;
+        cur = INV;
+    };
+    for (uint32_t base = first; base < end; base += WAVE) {
+        const uint32_t s = base + l;
+        const bool in = s < end;
+        const uint32_t r = in ? run[s] : INV;
+        const uint64_t se = in ? state_edges[s] : 0;
+        const uint64_t ps = in && cnt[s] ? ne[s] : 0;
+        if (in && run_sbeg[r] == s) tot[r] = moff[run_send[r]] - moff[s];
+        const uint32_t r0 = __shfl(r, 0, WAVE);
+        if (__ballot(in && r != r0) == 0) {
+            if (r0 != cur) { flush(); cur = r0; }
+            sum += se;
+            pe += ps;
+            continue;
+        }
+        flush();
+        const uint64_t a = wave_incl_scan_u64(se), b = wave_incl_scan_u64(ps);
+        const uint32_t prev = __shfl_up(r, 1, WAVE);
+        const uint64_t heads = __ballot(l == 0 || r != prev);
+        const uint32_t h = 63u - (uint32_t)__clzll((long long)(heads & ((2ull << l) - 1ull)));   // segment's first lane
+        const uint64_t a0 = wave_lane_u64(a, h ? h - 1 : 0), b0 = wave_lane_u64(b, h ? h - 1 : 0);
+        const bool last = l == WAVE - 1 || ((heads >> (l + 1)) & 1ull);
+        if (last && r != INV) add_run_totals(edges, parent_edges, r, a - (h ? a0 : 0), b - (h ? b0 : 0));
     }
-    sum = wave_sum_u64(sum);
-    pe = wave_sum_u64(pe);
-    if (l == 0) {
-        tot[r] = moff[e] - moff[b];
-        edges[r] = sum;
-        parent_edges[r] = pe;
-    }
+    flush();
 }
 
 // Zero the counts of states whose run does not advance this generation.
@@ -1658,11 +1688,13 @@ hipError_t launch_wl_states(const WLStatesArgs& a, uint32_t grid_cap, uint32_t w
 }
 
 hipError_t launch_run_totals(const uint64_t* moff, const uint64_t* state_edges, const uint32_t* cnt,
-                             const uint32_t* ne, const uint32_t* b, const uint32_t* e, uint32_t nruns, uint64_t* tot,
-                             uint64_t* edges, uint64_t* parent_edges, hipStream_t st) {
-    if (nruns == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_run_totals, dim3((nruns + 3) / 4), dim3(256), 0, st, moff, state_edges, cnt, ne, b, e, nruns,
-                       tot, edges, parent_edges);
+                             const uint32_t* ne, const uint32_t* run, uint32_t n, const uint32_t* b,
+                             const uint32_t* e, uint64_t* tot, uint64_t* edges, uint64_t* parent_edges,
+                             hipStream_t st) {
+    if (n == 0) return hipSuccess;
+    const uint32_t waves = (n + kTotalsChunk - 1) / kTotalsChunk;
+    hipLaunchKernelGGL(k_run_totals, dim3((waves + 3) / 4), dim3(256), 0, st, moff, state_edges, cnt, ne, run, n, b,
+                       e, tot, edges, parent_edges);
     return hipGetLastError();
 }
 

@@ -203,11 +203,13 @@ uint32_t wl_states_lds_per_wave(uint32_t max_ne, uint32_t max_nv, uint32_t A, bo
 // team: waves per state (1, 2, 4 or 8); with team 1, wpb states per workgroup.
 hipError_t launch_wl_states(const WLStatesArgs& a, uint32_t grid_cap, uint32_t wpb, uint32_t team, hipStream_t st);
 uint32_t wl_states_grid(uint32_t n, uint32_t team, uint32_t wpb, uint32_t grid_cap);
-// Per run (slot r, states [b[r], e[r])): tot[r] = its matches, edges[r] = its children's edges,
-// parent_edges[r] = the edges of its states with at least one match.
+// Per run (slot r, states [b[r], e[r]) of the n states, run[s] = the slot of state s): tot[r] = its
+// matches, edges[r] = its children's edges, parent_edges[r] = the edges of its states with at least
+// one match. The sums are added to: zero before the launch.
 hipError_t launch_run_totals(const uint64_t* moff, const uint64_t* state_edges, const uint32_t* cnt,
-                             const uint32_t* ne, const uint32_t* b, const uint32_t* e, uint32_t nruns, uint64_t* tot,
-                             uint64_t* edges, uint64_t* parent_edges, hipStream_t st);
+                             const uint32_t* ne, const uint32_t* run, uint32_t n, const uint32_t* b,
+                             const uint32_t* e, uint64_t* tot, uint64_t* edges, uint64_t* parent_edges,
+                             hipStream_t st);
 hipError_t launch_mask_counts(const uint32_t* run, const uint8_t* active, uint32_t n, uint32_t* cnt,
                               hipStream_t st);
 // Byte fill of [p, p + bytes) by a kernel: the engine clears its buffers with it (never
