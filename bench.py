@@ -165,10 +165,10 @@ def config2_line(ctx, steps, cpu_steps, threads, no_cpu):
            "canonical_states_per_s": round(c["canonical_states"] / wall, 1),
            "roofline": dominant(stats)}
     # atomic throughput of the state map: one 64-bit compare-and-swap insert (plus probes) per
-    # child state (one per event), all in k_dedup
-    dd = stats.get("k_dedup")
+    # child state (one per event), all in k_record
+    dd = stats.get("k_record")
     if dd and dd["total_ms"] > 0:
-        out["state_map"] = {"inserts": c["events"], "k_dedup_ms": round(dd["total_ms"], 4),
+        out["state_map"] = {"inserts": c["events"], "k_record_ms": round(dd["total_ms"], 4),
                             "inserts_per_s": round(c["events"] / (dd["total_ms"] * 1e-3), 1)}
     if not no_cpu:
         from oracle import pyoracle as po

@@ -132,48 +132,91 @@ __device__ inline uint32_t lanes_below(uint64_t mask) {
                                      __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }
 
-__device__ inline uint32_t wave_sum_u32(uint32_t v) {
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
-    return v;
+// Cross-lane steps by data-parallel moves (DPP within rows of 16 lanes, the row and half swaps of
+// gfx950 across them): a move is one VALU instruction with the latency of one, where a shuffle
+// (ds_bpermute) is a round trip through the LDS unit -- and these reductions are chains of 3 to 6
+// of them between the phases of every kernel here. A step reads only lanes of the reducing group,
+// all of which must be active.
+template <int CTRL, int ROWS = 0xF>
+__device__ __forceinline__ uint32_t dpp(uint32_t v) {          // 0 where no lane is read
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xF, true);
+}
+template <int CTRL, int ROWS = 0xF>
+__device__ __forceinline__ uint64_t dpp(uint64_t v) {
+    return ((uint64_t)dpp<CTRL, ROWS>((uint32_t)(v >> 32)) << 32) | dpp<CTRL, ROWS>((uint32_t)v);
+}
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E;               // quad permutations [1,0,3,2], [2,3,0,1]
+constexpr int kDppHalfMirror = 0x141, kDppMirror = 0x140;     // lane i <-> 7 - i, i <-> 15 - i
+constexpr int kDppRowShr = 0x110;                             // + n: from the lane n below in the row
+constexpr int kDppBcast15 = 0x142, kDppBcast31 = 0x143;       // a row's / half's last lane to the next
+
+// v of the other row of the pair (H = 16) or of the other half of the wave (H = 32): the swap of a
+// register with itself leaves the two rows' values in its two results, in that order for every lane.
+template <int H>
+__device__ __forceinline__ void swap_rows(uint32_t v, uint32_t& a, uint32_t& b) {
+    static_assert(H == 16 || H == 32, "rows of 16 or halves of 32 lanes");
+    if constexpr (H == 16) { const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false); a = r[0]; b = r[1]; }
+    else { const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false); a = r[0]; b = r[1]; }
+}
+template <int H>
+__device__ __forceinline__ void swap_rows(uint64_t v, uint64_t& a, uint64_t& b) {
+    uint32_t al, bl, ah, bh;
+    swap_rows<H>((uint32_t)v, al, bl);
+    swap_rows<H>((uint32_t)(v >> 32), ah, bh);
+    a = ((uint64_t)ah << 32) | al;
+    b = ((uint64_t)bh << 32) | bl;
 }
 
-__device__ inline uint32_t wave_max_u32(uint32_t v) {
-    for (int o = 32; o > 0; o >>= 1) { uint32_t w = __shfl_xor(v, o, WAVE); v = w > v ? w : v; }
+// f over the G consecutive lanes holding this one (f associative and commutative), to every lane.
+template <uint32_t G, class T, class F>
+__device__ __forceinline__ T group_reduce(T v, F f) {
+    static_assert(G == 8 || G == 16 || G == 32 || G == 64, "groups of 8 to 64 lanes");
+    v = f(v, dpp<kDppXor1>(v));
+    v = f(v, dpp<kDppXor2>(v));
+    v = f(v, dpp<kDppHalfMirror>(v));
+    if constexpr (G >= 16) v = f(v, dpp<kDppMirror>(v));
+    if constexpr (G >= 32) { T a, b; swap_rows<16>(v, a, b); v = f(a, b); }
+    if constexpr (G >= 64) { T a, b; swap_rows<32>(v, a, b); v = f(a, b); }
     return v;
 }
-
-__device__ inline uint64_t wave_sum_u64(uint64_t v) {
-    for (int o = 32; o > 0; o >>= 1) {
-        uint32_t lo = __shfl_xor((uint32_t)v, o, WAVE);
-        uint32_t hi = __shfl_xor((uint32_t)(v >> 32), o, WAVE);
-        v += ((uint64_t)hi << 32) | lo;
+template <uint32_t G, class T>
+__device__ __forceinline__ T group_sum(T v) { return group_reduce<G>(v, [](T x, T y) { return x + y; }); }
+template <uint32_t G>
+__device__ __forceinline__ uint32_t group_max(uint32_t v) {
+    return group_reduce<G>(v, [](uint32_t x, uint32_t y) { return x > y ? x : y; });
+}
+// Inclusive prefix sum over the G consecutive lanes holding this one; r is the lane's rank there.
+template <uint32_t G, class T>
+__device__ __forceinline__ T group_incl_scan(T v, uint32_t r) {
+    static_assert(G == 8 || G == 16 || G == 32 || G == 64, "groups of 8 to 64 lanes");
+    if constexpr (G == 8) {                       // a row holds two groups: keep to this one's lanes
+        const T a = dpp<kDppRowShr + 1>(v); v += r >= 1 ? a : T(0);
+        const T b = dpp<kDppRowShr + 2>(v); v += r >= 2 ? b : T(0);
+        const T c = dpp<kDppRowShr + 4>(v); v += r >= 4 ? c : T(0);
+    } else {
+        v += dpp<kDppRowShr + 1>(v);
+        v += dpp<kDppRowShr + 2>(v);
+        v += dpp<kDppRowShr + 4>(v);
+        v += dpp<kDppRowShr + 8>(v);
+        if constexpr (G >= 32) v += dpp<kDppBcast15, 0xA>(v);     // rows 1 and 3 take rows 0 and 2
+        if constexpr (G >= 64) v += dpp<kDppBcast31, 0xC>(v);     // the upper half takes the lower
     }
     return v;
 }
+
+__device__ inline uint32_t wave_sum_u32(uint32_t v) { return group_sum<WAVE>(v); }
+__device__ inline uint32_t wave_max_u32(uint32_t v) { return group_max<WAVE>(v); }
+__device__ inline uint64_t wave_sum_u64(uint64_t v) { return group_sum<WAVE>(v); }
 
 // Inclusive prefix sum across the wave.
-__device__ inline uint32_t wave_incl_scan_u32(uint32_t v) {
-    const uint32_t l = lane_id();
-    for (int o = 1; o < WAVE; o <<= 1) {
-        uint32_t w = __shfl_up(v, o, WAVE);
-        if (l >= (uint32_t)o) v += w;
-    }
-    return v;
-}
+__device__ inline uint32_t wave_incl_scan_u32(uint32_t v) { return group_incl_scan<WAVE>(v, lane_id()); }
 
 __device__ inline uint64_t wave_lane_u64(uint64_t v, uint32_t lane) {
     const uint32_t lo = __shfl((uint32_t)v, (int)lane, WAVE), hi = __shfl((uint32_t)(v >> 32), (int)lane, WAVE);
     return ((uint64_t)hi << 32) | lo;
 }
 
-__device__ inline uint64_t wave_incl_scan_u64(uint64_t v) {
-    const uint32_t l = lane_id();
-    for (int o = 1; o < WAVE; o <<= 1) {
-        const uint32_t lo = __shfl_up((uint32_t)v, o, WAVE), hi = __shfl_up((uint32_t)(v >> 32), o, WAVE);
-        if (l >= (uint32_t)o) v += ((uint64_t)hi << 32) | lo;
-    }
-    return v;
-}
+__device__ inline uint64_t wave_incl_scan_u64(uint64_t v) { return group_incl_scan<WAVE>(v, lane_id()); }
 
 // Exclusive prefix sum of a[0..n) in LDS, in place, by one wave; returns the total.
 __device__ __forceinline__ uint32_t wave_excl_scan_lds(uint32_t* a, uint32_t n) {
@@ -184,7 +227,7 @@ __device__ __forceinline__ uint32_t wave_excl_scan_lds(uint32_t* a, uint32_t n) 
         const uint32_t v = i < n ? a[i] : 0u;
         const uint32_t inc = wave_incl_scan_u32(v);
         if (i < n) a[i] = carry + inc - v;
-        carry += __shfl(inc, WAVE - 1, WAVE);
+        carry += (uint32_t)__builtin_amdgcn_readlane((int)inc, WAVE - 1);
     }
     wave_sync();
     return carry;
@@ -254,7 +297,7 @@ struct Team {
     __device__ uint32_t incl_scan(uint32_t v, uint32_t& total) const {
         const uint32_t inc = wave_incl_scan_u32(v);
         if constexpr (W == 1) {
-            total = __shfl(inc, WAVE - 1, WAVE);
+            total = (uint32_t)__builtin_amdgcn_readlane((int)inc, WAVE - 1);
             return inc;
         } else {
             const uint32_t w = threadIdx.x / WAVE;
@@ -274,7 +317,8 @@ struct Team {
     // The first member's value, to every member.
     __device__ uint64_t bcast(uint64_t v) const {
         if constexpr (W == 1) {
-            const uint32_t lo = __shfl((uint32_t)v, 0, WAVE), hi = __shfl((uint32_t)(v >> 32), 0, WAVE);
+            const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, 0);
+            const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), 0);
             return ((uint64_t)hi << 32) | lo;
         } else {
             if (r == 0) red[0] = v;
@@ -334,7 +378,7 @@ struct Team {
     }
 };
 
-// A sub-wave team: G consecutive lanes of one wave (G = 16 or 32) share one state, so a wave
+// A sub-wave team: G consecutive lanes of one wave (G = 8, 16 or 32) share one state, so a wave
 // works on 64 / G small states at once, each with its own workspace. The groups of a wave may
 // run different trip counts: every cross-lane step reads only the group's own lanes (shuffles
 // within width G, ballots masked to the group), and a group's lanes are all active at each such
@@ -342,7 +386,7 @@ struct Team {
 // the wave's (the groups share its program order).
 template <uint32_t G>
 struct SubTeam {
-    static_assert(G == 16 || G == 32, "sub-wave teams are 16 or 32 lanes");
+    static_assert(G == 8 || G == 16 || G == 32, "sub-wave teams are 8, 16 or 32 lanes");
     static constexpr uint32_t N = G;
     static constexpr uint32_t LANES = G;
     uint32_t r;             // rank in the team
@@ -356,30 +400,13 @@ struct SubTeam {
     __device__ uint32_t shfl(uint32_t v, uint32_t u) const { return __shfl(v, (int)u, (int)G); }
     __device__ uint32_t read_lane(uint32_t v, uint32_t u) const { return __shfl(v, (int)u, (int)G); }
     __device__ uint64_t ballot(bool b) const { return (__ballot(b) >> base) & ((1ull << G) - 1ull); }
-    __device__ uint32_t sum(uint32_t v) const {
-        for (uint32_t o = G / 2; o > 0; o >>= 1) v += __shfl_xor(v, (int)o, WAVE);
-        return v;
-    }
-    __device__ uint64_t sum64(uint64_t v) const {
-        for (uint32_t o = G / 2; o > 0; o >>= 1) {
-            const uint32_t lo = __shfl_xor((uint32_t)v, (int)o, WAVE);
-            const uint32_t hi = __shfl_xor((uint32_t)(v >> 32), (int)o, WAVE);
-            v += ((uint64_t)hi << 32) | lo;
-        }
-        return v;
-    }
-    __device__ uint32_t max(uint32_t v) const {
-        for (uint32_t o = G / 2; o > 0; o >>= 1) { const uint32_t w = __shfl_xor(v, (int)o, WAVE); v = w > v ? w : v; }
-        return v;
-    }
+    __device__ uint32_t sum(uint32_t v) const { return group_sum<G>(v); }
+    __device__ uint64_t sum64(uint64_t v) const { return group_sum<G>(v); }
+    __device__ uint32_t max(uint32_t v) const { return group_max<G>(v); }
     __device__ bool any(bool b) const { return ballot(b) != 0; }
     __device__ uint32_t incl_scan(uint32_t v, uint32_t& total) const {
-        for (uint32_t o = 1; o < G; o <<= 1) {
-            const uint32_t w = __shfl_up(v, o, (int)G);
-            if (r >= o) v += w;
-        }
-        total = __shfl(v, (int)(G - 1), (int)G);
-        return v;
+        total = group_sum<G>(v);
+        return group_incl_scan<G>(v, r);
     }
     __device__ uint64_t bcast(uint64_t v) const {
         const uint32_t lo = __shfl((uint32_t)v, 0, (int)G), hi = __shfl((uint32_t)(v >> 32), 0, (int)G);

@@ -10,6 +10,7 @@
 
 #include "hgx_engine.hpp"
 #include "hgx_kernels.hpp"
+#include "hgx_wl_small.hpp"
 
 namespace hgx {
 
@@ -232,6 +233,34 @@ constexpr uint32_t kExpandEdges[kExpandClasses] = {32, 64, 128, 512, 2048, 0xFFF
 static_assert(kExpandClasses == kTuneExpandClasses, "one tuned shape per expansion size class");
 static_assert(sizeof(kClassEdges) / sizeof(kClassEdges[0]) == kTuneJoinClasses, "one tuned shape per join size class");
 
+// Launch shape of k_expand_small: lanes per child, waves per workgroup, workgroups per CU.
+struct SmallShape {
+    uint32_t lds, lanes, wpb, grid;
+};
+// Fewer lanes per child mean fewer instructions per child (the steps between phases are a wave's,
+// whatever it holds) but more LDS per wave and a longer child: 16 lanes up to 64 edges, 32 up to 128,
+// then a wave. Batched workload, k_expand of a pass in its class with the others fixed: up to 32
+// edges 8 / 16 / 32 lanes 5.69 / 5.68 / 6.24 ms, up to 64 6.67 / 5.67 / 6.37, up to 128 - / 5.68 /
+// 5.62 (60 results of 3 to 80 edges 1.43 / 1.29). 8 lanes where a launch is long and its workspaces
+// small enough that a CU still holds over a hundred children: 10.3 M children of 29 labels 8.4 -> 7.0
+// ms, with 32 workgroups per CU 6.5 (16 lanes 7.6); 0.29 M 0.49 -> 0.53, so not there. Waves per
+// workgroup as many of 4, 2, 1 as leave a CU the most waves.
+SmallShape small_shape(const ExpandArgs& a, uint32_t K, uint32_t forced, uint32_t max_lds, uint32_t A) {
+    SmallShape s{expand_small_lds(a.max_child_ne, a.max_nextv, A), 0, 1, 8};
+    const bool lng = a.n_items >= (1u << 20);
+    s.lanes = a.max_child_ne <= 64 ? (lng && a.max_nextv <= 32 ? 8u : 16u) : a.max_child_ne <= 128 ? 32u : 64u;
+    if (forced) s.lanes = forced;
+    while (s.lanes < 64 && (K > s.lanes || (uint64_t)s.lds * (64 / s.lanes) > max_lds)) s.lanes *= 2;
+    const uint32_t wave = s.lds * (64 / s.lanes);
+    uint32_t held = 0;
+    for (uint32_t w : {4u, 2u, 1u}) {
+        const uint32_t waves = max_lds / (wave * w) * w;
+        if (waves > held) { held = waves; s.wpb = w; }
+    }
+    s.grid = (lng ? 32u : 8u) * 4u / s.wpb;
+    return s;
+}
+
 // A stride near n / golden ratio and coprime to n, so i -> i * stride mod n visits 0..n-1 once
 // each, consecutive i far apart (1 for n <= 2: in order).
 uint32_t coprime_stride(uint32_t n) {
@@ -441,7 +470,7 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
                     if (F_e_[i] == F_b_[i]) continue;
                     int k = 0;
                     while (r.ne_bound > kClassEdges[k]) ++k;
-                    ExpandClass& x = cls[k];
+                        ExpandClass& x = cls[k];
                     x.ne = std::max(x.ne, r.ne_bound);
                     x.nextv = std::max(x.nextv, r.nv_bound);
                     x.rb.push_back(F_b_[i]);
@@ -695,7 +724,6 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
     std::vector<uint8_t> r_depth, r_ar;
     std::vector<RootCopy> r_copy;
     ExpandClass cls[kExpandClasses];            // host range lists of the expand launches
-    std::vector<RunEvents> rev;                 // per-run child ranges for k_run_events
     const uint32_t nC = (uint32_t)M + NR;
     if (nC) {
         C = std::make_shared<DevGen>(pool_);
@@ -795,14 +823,12 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
                 x.rpre.push_back((uint32_t)x.n);
             }
             const uint64_t bytes = M * (8ull + 2ull * K) + parent_edges * (4ull * F_->v.A + 2) +
-                                   EC * (4ull * A + 2) + M * (28ull + 8ull * lstride) + M * 24ull;
-            uint16_t* tcnt = dalloc<uint16_t>(tmp, M);   // per child: causal triples, for k_run_events
+                                   EC * (4ull * A + 2) + M * 8ull;
             for (int k = 0; k < kExpandClasses; ++k) {
                 ExpandClass& x = cls[k];
                 if (!x.n) continue;
                 ExpandArgs ea{};
                 ea.P = F_->v; ea.C = v; ea.M = mv; ea.E = C->ev; ea.runs = d_runs_; ea.ctr = d_ctr_;
-                ea.tcnt = tcnt;
                 ea.max_child_ne = std::max(1u, std::min(x.ne, max_ne));
                 ea.max_nextv = std::max(1u, std::min(x.nextv, max_nextv));
                 ea.max_nv = std::max(1u, std::min(ea.max_nextv, ea.max_child_ne * A));
@@ -814,6 +840,14 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
                     up(d_r, x.rb.data(), x.rb.size(), st);
                     up(d_r + x.rb.size(), x.rpre.data(), x.rpre.size(), st);
                     ea.rb = d_r; ea.rpre = d_r + x.rb.size(); ea.nrange = (uint32_t)x.rb.size();
+                }
+                if (ea.lean && ea.max_child_ne <= kSmallMaxEdges && ea.max_nextv <= kSmallMaxLabels &&
+                    ctx_->expand_team <= 1) {
+                    const SmallShape sh = small_shape(ea, K, ctx_->expand_lanes, ctx_->max_lds, A);
+                    ea.lds_per_wave = sh.lds;
+                    timed(ctx_, st, "k_expand", (uint64_t)((double)bytes * x.n / M), x.n,
+                          [&] { return launch_expand_small(ea, ctx_->num_cu * sh.grid, sh.wpb, sh.lanes, st); }, k);
+                    continue;
                 }
                 // Team: one wave per child while a CU still holds several workspaces, else the
                 // workgroup's waves share one child (a CU holds 160 KiB of LDS).
@@ -837,16 +871,10 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
                 timed(ctx_, st, "k_expand", (uint64_t)((double)bytes * x.n / M), x.n,
                       [&] { return launch_expand(ea, gcap, wpb_e, team, st, lanes); }, k);
             }
-            timed(ctx_, st, "k_dedup", M * 12ull + M * 8ull, M,
-                  [&] { return launch_dedup(v, (uint32_t)M, d_runs_, d_ctr_, st); });
-            // each run's event counters from its children's records: one add per run
-            for (uint32_t i = 0; i < nF; ++i)                // items of at most 4,096 children
-                for (uint64_t b = cb[i]; b < ce[i]; b += 4096)
-                    rev.push_back(RunEvents{F_runs_[i]->slot, (uint32_t)b,
-                                            (uint32_t)std::min<uint64_t>(ce[i], b + 4096)});
-            RunEvents* d_rev = dalloc<RunEvents>(tmp, rev.size());
-            up(d_rev, rev.data(), rev.size(), st);
-            HIP_TRY(launch_run_events(d_rev, (uint32_t)rev.size(), C->ev, tcnt, d_ctr_, st));
+            ExpandArgs ra{};
+            ra.P = F_->v; ra.C = v; ra.M = mv; ra.E = C->ev; ra.runs = d_runs_; ra.ctr = d_ctr_;
+            timed(ctx_, st, "k_record", M * (8ull + 2ull * K) + M * (28ull + 8ull * lstride) + M * 24ull + M * 20ull, M,
+                  [&] { return launch_record(ra, (uint32_t)M, st); });
         }
 
         // new roots: uploaded (host inputs) or copied on the device (prepared inputs), then

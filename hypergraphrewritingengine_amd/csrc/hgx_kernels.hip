@@ -2,9 +2,10 @@
 //
 //   k_match<false>   SCAN -> EXPAND -> SINK join, counting matches per state
 //   k_match<true>    the same join, writing match records in the deterministic order
-//   k_expand         rewrite + WL hash + event + causal emission, one team per child state
-//   k_dedup          each child's hash into its request's state map
-//   k_run_events     a generation's event and causal counters, summed per request
+//   k_expand         rewrite + WL hash, one team per child state
+//                    (k_expand_small: small children of one arity)
+//   k_record         each child's event, causal masks and records, its hash into its request's
+//                    state map, and the request's counters
 //   k_branchial      sibling-event overlap pairs, one wave per parent state (k_brl_*: the
 //                    sorted per-edge lists for parents above 128 edges)
 //   k_wl_states      WL hash of given states (roots, and the hgx_wl_hash_batch entry point)
@@ -23,6 +24,7 @@
 #include "hgx_device.hpp"
 #include "hgx_kernels.hpp"
 #include "hgx_wl.hpp"
+#include "hgx_wl_small.hpp"
 
 namespace hgx {
 
@@ -706,7 +708,7 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W, W == 1 ? 4 : 1) void k_match
 
 
 // ------------------------------------------------------------------------------------------
-// Rewrite + hash + dedup + event + causal, one wave per child (Rewriter::apply,
+// Rewrite + hash, one team per child, then the children's records (Rewriter::apply,
 // hypergraph/src/rewriter.cpp:11-205, with hgcommon rewrite semantics rewrite_core.hpp:53-87).
 // ------------------------------------------------------------------------------------------
 
@@ -746,7 +748,6 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W, W == 1 ? 4 : 1) void k_expan
     if constexpr (GWS) my = a.scratch + ((size_t)blockIdx.x * tpb + w) * a.lds_per_wave;
     else my = lds + (size_t)w * a.lds_per_wave;
     const TM tm((uint64_t*)(my + a.lds_per_wave - 64));   // a wave team's reduction words: the last 64 bytes
-    const uint32_t l = tm.lane();
     const uint32_t PA = a.P.A, A = a.C.A;                  // parent / child vertex strides
     const WLSizes z = expand_sizes(a.max_child_ne, a.max_nv, a.max_nextv, A, a.lean != 0);
     WLSpace s;
@@ -781,8 +782,7 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W, W == 1 ? 4 : 1) void k_expan
         const uint32_t par = a.M.parent[c];
         const uint32_t rid = a.M.rule[c];
         const uint32_t run = a.P.run[par];
-        DRun* RN = &a.runs[run];
-        const DRule& R = RN->rules[rid];
+        const DRule& R = a.runs[run].rules[rid];
         const uint32_t nl = R.n_lhs, nr = R.n_rhs;
         const uint32_t pne = a.P.ne[par];
         const uint64_t peo = a.P.eoff[par];
@@ -791,18 +791,6 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W, W == 1 ? 4 : 1) void k_expan
         const uint32_t pdep = a.P.depth[par];
         const uint32_t step = pdep + 1;                       // generation of the child
         const uint16_t* q = a.M.q + (size_t)c * a.M.K;
-        // Causal inputs, fetched now so their latency hides under the rewrite and the hash:
-        // lane t < nl holds the producer generation of consumed edge t (0: none) and that
-        // producer's causal-ancestor mask from the parent's lineage table.
-        uint32_t ps_t = 0;
-        uint64_t anc_t = 0;
-        if (l < nl) {
-            ps_t = a.P.ps[peo + q[l]];
-            if (ps_t) anc_t = a.P.lanc[(size_t)par * a.P.lstride + ps_t - 1];
-        }
-
-        if (a.E.cps && l < nl) a.E.cps[(size_t)c * a.E.cK + l] = (uint8_t)ps_t;
-
         // Parent edges minus the consumed ones, order kept (SparseBitset::derive).
         uint32_t kept = 0;
         for (uint32_t base = 0; base < pne; base += TM::N) {
@@ -864,90 +852,121 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W, W == 1 ? 4 : 1) void k_expan
         s.nV = nv;
         tm.sync();
         const uint64_t h = wl_hash_team(s, tm);
-
-        // Causal: one triple per consumed edge with a producer; the producers are events of
-        // this lineage, named by their generation (rewriter.cpp:121-191,
-        // causal_graph.cpp:187-234). Transitive reduction: (P, C) is redundant exactly when P
-        // is a causal ancestor of another producer of C. Every lane computes the same masks
-        // from the nl lanes holding the consumed edges' producers.
-        uint64_t prod = 0, anc_c = 0, others = 0;
-        for (uint32_t u = 0; u < nl; ++u) {
-            const uint32_t pu = tm.shfl(ps_t, u);
-            const uint64_t au = ((uint64_t)tm.shfl((uint32_t)(anc_t >> 32), u) << 32) |
-                                tm.shfl((uint32_t)anc_t, u);
-            if (pu) {
-                prod |= 1ull << pu;
-                anc_c |= (1ull << pu) | au;
-                if (pu != ps_t) others |= au;
-            }
-        }
-        const bool rec_causal = (RN->flags & 0x1u) != 0;
-        const bool drop = (RN->flags & 0x100u) && l < nl && ps_t && ((others >> ps_t) & 1ull);
-        const uint64_t dropped = tm.ballot(drop);
-        uint64_t tr = prod;
-        for (uint32_t u = 0; u < nl; ++u) {
-            const uint32_t pu = tm.shfl(ps_t, u);
-            if ((dropped >> u) & 1ull) tr &= ~(1ull << pu);
-        }
-        const uint32_t triples = (uint32_t)__popcll(tm.ballot(l < nl && ps_t != 0));
-        const uint32_t triples_tr = (uint32_t)__popcll(tm.ballot(l < nl && ps_t != 0 && ((tr >> ps_t) & 1ull)));
-        if (!rec_causal) { prod = 0; tr = 0; anc_c = 0; }
-
-        // Identity and bookkeeping (the team's first lane): the child's record and its event.
-        const uint32_t ev_id = RN->ev_base + (c - RN->child_begin);
-        const uint32_t child_sid = RN->n_roots + ev_id;
-        if (tm.leader()) {
-            a.C.run[c] = run;
-            a.C.ne[c] = cne;
-            a.C.nextv[c] = nextv;
-            a.C.sid[c] = child_sid;
-            a.C.hash[c] = h;
-            a.C.depth[c] = (uint8_t)step;
-            a.E.in_state[c] = a.P.sid[par];
-            a.E.rule[c] = rid;
-            a.E.prod[c] = prod;
-            a.E.tr[c] = tr;
-            // the run's counters are summed from these by k_run_events, not added here
-            a.tcnt[c] = rec_causal ? (uint16_t)(triples | (triples_tr << 8)) : (uint16_t)0;
-        }
-        // Lineage table of the child: the parent's, then this event's ancestor mask.
-        {
-            const uint64_t* plan = a.P.lanc + (size_t)par * a.P.lstride;
-            uint64_t* clan = a.C.lanc + (size_t)c * a.C.lstride;
-            for (uint32_t t = tm.r; t < step; t += TM::N) clan[t] = (t + 1 == step) ? anc_c : plan[t];
-        }
+        if (tm.leader()) a.C.hash[c] = h;              // the child's other records: k_record
         tm.sync();
     }
 }
 
-// A generation's event counters per run (items of at most a few thousand of a run's children
-// [cb, ce), one wave each): events, causal triples and pairs with and without transitive
-// reduction, from the per-child records k_expand wrote -- one add per counter and item instead
-// of adds from every team.
-__global__ void k_run_events(const RunEvents* items, uint32_t n, const uint64_t* prod, const uint64_t* tr,
-                             const uint16_t* tcnt, uint64_t* ctr) {
-    const uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE, l = lane_id();
-    if (i >= n) return;
-    const RunEvents it = items[i];
-    uint64_t triples = 0, pairs = 0, pairs_tr = 0, triples_tr = 0;
-    for (uint32_t c = it.cb + l; c < it.ce; c += WAVE) {
-        const uint32_t t = tcnt[c];
-        triples += t & 0xFFu;
-        triples_tr += t >> 8;
-        pairs += (uint64_t)__popcll(prod[c]);
-        pairs_tr += (uint64_t)__popcll(tr[c]);
-    }
-    triples = wave_sum_u64(triples);
-    triples_tr = wave_sum_u64(triples_tr);
-    pairs = wave_sum_u64(pairs);
-    pairs_tr = wave_sum_u64(pairs_tr);
-    if (l == 0) {                                    // a large run is split over several items
-        unsigned long long* row = (unsigned long long*)(ctr + (size_t)it.slot * CTR_N);
-        atomicAdd(&row[CTR_EVENTS], (unsigned long long)(it.ce - it.cb));
-        if (triples) atomicAdd(&row[CTR_TRIPLES], (unsigned long long)triples);
-        if (pairs) atomicAdd(&row[CTR_PAIRS], (unsigned long long)pairs);
-        if (pairs_tr) atomicAdd(&row[CTR_PAIRS_TR], (unsigned long long)pairs_tr);
-        if (triples_tr) atomicAdd(&row[CTR_TRIPLES_TR], (unsigned long long)triples_tr);
+// k_expand for small children of one arity (ExpandArgs::small): the same records, with the hash of
+// hgx_wl_small.hpp. Labels are bytes, so the rewrite leaves its edges in LDS as the hash reads them;
+// a kept edge's place is its position less the consumed positions below it (two words of bits), so
+// the copy needs no compaction and its loads do not wait for each other.
+template <uint32_t UA, uint32_t G>
+__global__ __launch_bounds__(256, 5) void k_expand_small(ExpandArgs a) {
+    using TM = typename TeamSel<1, G>::type;
+    extern __shared__ uint8_t lds[];
+    const uint32_t tpb = (blockDim.x / WAVE) * (WAVE / G);                 // teams per workgroup
+    const uint32_t w = threadIdx.x / G;
+    const TM tm(nullptr);
+    const uint32_t l = tm.r;
+    const uint32_t PA = UA ? UA : a.P.A, A = UA ? UA : a.C.A;              // parent / child vertex strides
+    SmallSpace s;
+    small_bind(s, lds + (size_t)w * a.lds_per_wave, SmallSizes::make(a.max_child_ne, a.max_nextv, A), A);
+
+    // Children in chunks of a.chunk consecutive ones, dealt round-robin to the teams: 2 keep a
+    // parent's neighbouring children on one team, 1 where the launch has a team for every child.
+    const uint32_t chunk = a.chunk;
+    const uint32_t gw = xcd_block() * tpb + w, nw = gridDim.x * tpb;
+    uint32_t rr = 0;
+    for (uint32_t lc = gw * chunk, at = 0; lc < a.n_items;) {
+        uint32_t c = lc;
+        if (a.nrange) {
+            if (at == 0) {                                     // a new chunk: find its range
+                uint32_t lo = 0, hi = a.nrange;
+                while (hi - lo > 1) { const uint32_t mid = (lo + hi) >> 1; if (a.rpre[mid] <= lc) lo = mid; else hi = mid; }
+                rr = lo;
+            }
+            while (lc >= a.rpre[rr + 1]) ++rr;
+            c = a.rb[rr] + (lc - a.rpre[rr]);
+        }
+        if (++at == chunk) { at = 0; lc += (nw - 1) * chunk + 1; } else ++lc;
+        const uint32_t par = a.M.parent[c];
+        const uint32_t rid = a.M.rule[c];
+        const uint64_t ceo = a.C.eoff[c];
+        const uint32_t q_t = l < a.M.K ? a.M.q[(size_t)c * a.M.K + l] : 0u;     // consumed position l
+        const uint32_t run = a.P.run[par];
+        const uint32_t pne = a.P.ne[par];
+        const uint64_t peo = a.P.eoff[par];
+        const uint32_t fresh_base = a.P.nextv[par];
+        const uint32_t step = a.P.depth[par] + 1u;            // generation of the child
+        const DRule& R = a.runs[run].rules[rid];
+        const uint32_t nl = R.n_lhs, nr = R.n_rhs;
+        const uint32_t ua = UA ? UA : R.la[0];
+        const uint32_t cne = pne - nl + nr, kept = pne - nl;
+        uint64_t used[4] = {0, 0, 0, 0};                       // consumed positions (below 256)
+        for (uint32_t t = 0; t < nl; ++t) {
+            const uint32_t q = tm.shfl(q_t, t);
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k)
+                if ((q >> 6) == k) used[k] |= 1ull << (q & 63u);
+        }
+        // parent edges minus the consumed ones, order kept (SparseBitset::derive)
+        for (uint32_t i = l; i < pne; i += TM::N) {
+            const uint32_t iw = i >> 6;
+            uint32_t below = 0;
+            bool keep = true;
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k) {
+                const uint64_t low = iw > k ? ~0ull : iw == k ? (1ull << (i & 63u)) - 1ull : 0ull;
+                below += (uint32_t)__popcll(used[k] & low);
+                if (iw == k) keep = !((used[k] >> (i & 63u)) & 1ull);
+            }
+            if (!keep) continue;
+            const uint32_t pos = i - below;
+            if constexpr (UA == 2) {
+                const uint2 v = ((const uint2*)a.P.ev)[peo + i];
+                ((uint2*)a.C.ev)[ceo + pos] = v;
+                ((uint16_t*)s.ev)[pos] = (uint16_t)(v.x | (v.y << 8));
+            } else {
+                for (uint32_t k = 0; k < A; ++k) {
+                    const uint32_t v = k < PA ? a.P.ev[(peo + i) * PA + k] : 0u;
+                    a.C.ev[(ceo + pos) * A + k] = v;
+                    if (k < ua) s.ev[pos * ua + k] = (uint8_t)v;
+                }
+            }
+            a.C.ar[ceo + pos] = (uint8_t)ua;
+            a.C.ps[ceo + pos] = a.P.ps[peo + i];
+        }
+        // produced edges in RHS order; fresh vertices ascending by variable
+        // (assign_fresh_consecutive / resolve_rhs_vertices, rewrite_core.hpp:53-87)
+        for (uint32_t base = 0; base < nr; base += TM::N) {
+            const uint32_t t = base + l;
+            const uint32_t pos = kept + t;
+            for (uint32_t k = 0; k < A; ++k) {
+                uint32_t v = 0, se = 0, var = 0;
+                const bool in = t < nr && k < ua;
+                if (in) {
+                    var = R.rv[t][k];
+                    se = R.var_src_edge[var];
+                }
+                const uint32_t q = tm.shfl(q_t, se);           // every lane of the team takes part
+                if (in) {
+                    if (R.lhs_mask & (1u << var)) v = a.P.ev[(peo + q) * PA + R.var_src_pos[var]];
+                    else v = fresh_base + __popc(R.new_mask & ((1u << var) - 1u));
+                    s.ev[pos * ua + k] = (uint8_t)v;
+                }
+                if (t < nr) a.C.ev[(ceo + pos) * A + k] = v;
+            }
+            if (t < nr) {
+                a.C.ar[ceo + pos] = (uint8_t)ua;
+                a.C.ps[ceo + pos] = (uint8_t)step;
+            }
+        }
+        tm.sync();
+        const uint32_t nextv = fresh_base + R.n_new;
+        const uint64_t h = wl_hash_small<UA>(s, tm, cne, nextv, ua);
+        if (tm.leader()) a.C.hash[c] = h;              // the child's other records: k_record
+        tm.sync();
     }
 }
 
@@ -1073,13 +1092,6 @@ hipError_t launch_plan_check(const uint64_t* tot, const uint64_t* want, const ui
     return hipGetLastError();
 }
 
-hipError_t launch_run_events(const RunEvents* items, uint32_t n, const EventView& E, const uint16_t* tcnt,
-                             uint64_t* ctr, hipStream_t st) {
-    if (!n) return hipSuccess;
-    hipLaunchKernelGGL(k_run_events, dim3((n + 3) / 4), dim3(256), 0, st, items, n, E.prod, E.tr, tcnt, ctr);
-    return hipGetLastError();
-}
-
 // ------------------------------------------------------------------------------------------
 // Branchial pairs of parents above BR_MAX_EDGES edges. Every (consumed edge slot, match) of such
 // a parent becomes one 64-bit key (slot << 32 | match); sorted, the keys of one slot are its consuming
@@ -1175,47 +1187,135 @@ hipError_t launch_brl(const BrListArgs& a, int phase, hipStream_t st) {
     return hipGetLastError();
 }
 
-// State identity (Hypergraph::create_or_get_canonical_state, hypergraph/src/hypergraph.cpp:154-254):
-// every child's hash into its request's state map, one lane per child, after k_expand -- so no
-// wave of k_expand waits on a global compare-and-swap chain. A key inserted first counts a
-// canonical state and adds to the fingerprint.
+// The records of a generation's children, one lane per child, after k_expand: the event, its causal
+// masks and lineage table, the child's own record, and its identity -- its hash into its request's
+// state map (Hypergraph::create_or_get_canonical_state, hypergraph/src/hypergraph.cpp:154-254) --
+// with the request's counters. Apart from k_expand because none of it needs a team: there a few lanes
+// of each team did it while the hash's registers were live, and its values lived through the hash.
 //
-// Device-scope atomics are performed beyond the L2 and each moves a whole request over the
-// fabric (measured on gfx950: 64 bytes per compare-and-swap, taken or not, 32 per add), and the
-// children of one generation that hash alike all find the slot empty before any of them claims
-// it. So a lane whose (request, hash) equals a lower lane's in the wave leaves the insert to that
-// lane, and when the wave's lanes belong to one request (the usual case: a request's children
-// are contiguous) the canonical count and fingerprint are summed over the wave and added once.
-__global__ void k_dedup(GenView C, uint32_t n, DRun* runs, uint64_t* ctr) {
-    const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool valid = c < n;
-    const uint32_t run = valid ? C.run[c] : 0xFFFFFFFFu;
-    const uint64_t h = valid ? C.hash[c] : 0;
-    const uint32_t lane = lane_id();
-    bool dup = false;
-    for (int k = 0; k < WAVE; ++k) {
-        const uint64_t hk = __shfl(h, k, WAVE);
-        const uint32_t rk = __shfl(run, k, WAVE);
-        dup |= k < (int)lane && hk == h && rk == run;
-    }
-    const bool fresh = valid && !dup && map_insert(&runs[run], h);
-    const uint32_t r0 = __shfl(run, 0, WAVE);
-    if (__ballot(valid && run != r0) == 0) {
-        const uint64_t nfresh = (uint64_t)__popcll(__ballot(fresh));
-        const uint64_t fp = wave_sum_u64(fresh ? mix64(h) : 0ull);
-        if (lane == 0 && nfresh) {
-            atomicAdd((unsigned long long*)&ctr[(size_t)r0 * CTR_N + CTR_CANON], (unsigned long long)nfresh);
-            atomicAdd((unsigned long long*)&ctr[(size_t)r0 * CTR_N + CTR_FINGERPRINT], (unsigned long long)fp);
+// Causal: one triple per consumed edge with a producer; the producers are events of this lineage,
+// named by their generation (rewriter.cpp:121-191, causal_graph.cpp:187-234). Transitive reduction: a
+// producer is redundant exactly when it is a causal ancestor of another one (an ancestor mask never
+// holds the event's own generation, so of any one).
+//
+// Device-scope atomics are performed beyond the L2 and each moves a whole request over the fabric
+// (measured on gfx950: 64 bytes per compare-and-swap, taken or not, 32 per add), and the children of
+// one generation that hash alike all find the slot empty before any of them claims it. So a lane
+// whose (request, hash) equals a lower lane's in the wave leaves the insert to that lane, and a wave
+// keeps the counters of the run its lanes hold (a run's children are contiguous) in registers over
+// all of its children, adding them when the run changes.
+constexpr uint32_t kRecordWaves = 4096;   // at most, so one large run is added to by as many waves
+__global__ __launch_bounds__(256) void k_record(ExpandArgs a, uint32_t n, uint32_t chunk) {
+    const uint32_t l = lane_id();
+    const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
+    const uint32_t first = wave * chunk, end = min(n, first + chunk);
+    uint32_t cur = INV;                                   // the run whose counters the lanes hold
+    uint32_t events = 0, canon = 0, triples = 0, triples_tr = 0, pairs = 0, pairs_tr = 0;
+    uint64_t fp = 0;
+    auto flush = [&] {
+        if (cur != INV) {
+            const uint32_t ev = wave_sum_u32(events);
+            const uint32_t cn = wave_sum_u32(canon);
+            const uint32_t t = wave_sum_u32(triples), tt = wave_sum_u32(triples_tr);
+            const uint32_t pr = wave_sum_u32(pairs), pt = wave_sum_u32(pairs_tr);
+            const uint64_t f = wave_sum_u64(fp);
+            if (l == 0) {
+                unsigned long long* row = (unsigned long long*)(a.ctr + (size_t)cur * CTR_N);
+                atomicAdd(&row[CTR_EVENTS], (unsigned long long)ev);
+                if (cn) {
+                    atomicAdd(&row[CTR_CANON], (unsigned long long)cn);
+                    atomicAdd(&row[CTR_FINGERPRINT], (unsigned long long)f);
+                }
+                if (t) atomicAdd(&row[CTR_TRIPLES], (unsigned long long)t);
+                if (tt) atomicAdd(&row[CTR_TRIPLES_TR], (unsigned long long)tt);
+                if (pr) atomicAdd(&row[CTR_PAIRS], (unsigned long long)pr);
+                if (pt) atomicAdd(&row[CTR_PAIRS_TR], (unsigned long long)pt);
+            }
         }
-    } else if (fresh) {
-        atomicAdd((unsigned long long*)&ctr[(size_t)run * CTR_N + CTR_CANON], 1ull);
-        atomicAdd((unsigned long long*)&ctr[(size_t)run * CTR_N + CTR_FINGERPRINT], (unsigned long long)mix64(h));
+        events = canon = triples = triples_tr = pairs = pairs_tr = 0;
+        fp = 0;
+    };
+    for (uint32_t base = first; base < end; base += WAVE) {
+        const uint32_t c = base + l;
+        const bool in = c < end;
+        uint32_t run = INV, t_n = 0, tt_n = 0, p_n = 0, pt_n = 0;
+        uint64_t h = 0;
+        if (in) {
+            const uint32_t par = a.M.parent[c], rid = a.M.rule[c];
+            h = a.C.hash[c];
+            run = a.P.run[par];
+            const uint32_t pne = a.P.ne[par], nextv = a.P.nextv[par], in_state = a.P.sid[par];
+            const uint64_t peo = a.P.eoff[par];
+            const uint32_t step = a.P.depth[par] + 1u;    // generation of the child
+            const DRun& RN = a.runs[run];
+            const DRule& R = RN.rules[rid];
+            const uint32_t nl = R.n_lhs, cne = pne - nl + R.n_rhs;
+            const uint16_t* q = a.M.q + (size_t)c * a.M.K;
+            const uint64_t* plan = a.P.lanc + (size_t)par * a.P.lstride;
+            uint64_t prod = 0, anc = 0;                   // producers' generations; their ancestors
+            for (uint32_t t = 0; t < nl; ++t) {
+                const uint32_t ps = a.P.ps[peo + q[t]];
+                if (a.E.cps) a.E.cps[(size_t)c * a.E.cK + t] = (uint8_t)ps;
+                if (ps) {
+                    prod |= 1ull << ps;
+                    anc |= plan[ps - 1];
+                    ++t_n;
+                }
+            }
+            uint64_t tr = (RN.flags & 0x100u) ? prod & ~anc : prod;
+            anc |= prod;
+            if (RN.flags & 0x1u) {
+                for (uint32_t t = 0; t < nl; ++t) tt_n += (uint32_t)((tr >> a.P.ps[peo + q[t]]) & 1ull);
+            } else {
+                prod = 0; tr = 0; anc = 0; t_n = 0;
+            }
+            p_n = (uint32_t)__popcll(prod);
+            pt_n = (uint32_t)__popcll(tr);
+            const uint32_t ev_id = RN.ev_base + (c - RN.child_begin);
+            a.C.run[c] = run;
+            a.C.ne[c] = cne;
+            a.C.nextv[c] = nextv + R.n_new;
+            a.C.sid[c] = RN.n_roots + ev_id;
+            a.C.depth[c] = (uint8_t)step;
+            a.E.in_state[c] = in_state;
+            a.E.rule[c] = rid;
+            a.E.prod[c] = prod;
+            a.E.tr[c] = tr;
+            // lineage table: the parent's, then this event's ancestor mask
+            uint64_t* clan = a.C.lanc + (size_t)c * a.C.lstride;
+            for (uint32_t t = 0; t + 1 < step; ++t) clan[t] = plan[t];
+            clan[step - 1] = anc;
+        }
+        bool dup = false;
+        for (int k = 0; k < WAVE - 1; ++k) {
+            const uint32_t hl = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)h, k);
+            const uint32_t hh = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(h >> 32), k);
+            const uint32_t rk = (uint32_t)__builtin_amdgcn_readlane((int)run, k);
+            dup |= k < (int)l && hl == (uint32_t)h && hh == (uint32_t)(h >> 32) && rk == run;
+        }
+        const bool fresh = in && !dup && map_insert(&a.runs[run], h);
+        const uint64_t f = fresh ? mix64(h) : 0ull;
+        for (uint64_t left = __ballot(in); left;) {       // the runs among the lanes, usually one
+            const uint32_t r0 = (uint32_t)__builtin_amdgcn_readlane((int)run, (int)__builtin_ctzll(left));
+            const bool mine = run == r0;
+            if (r0 != cur) { flush(); cur = r0; }
+            if (mine) {
+                events += 1;
+                canon += fresh ? 1u : 0u;
+                fp += f;
+                triples += t_n; triples_tr += tt_n; pairs += p_n; pairs_tr += pt_n;
+            }
+            left &= ~__ballot(mine);
+        }
     }
+    flush();
 }
 
-hipError_t launch_dedup(const GenView& C, uint32_t n, DRun* runs, uint64_t* ctr, hipStream_t st) {
+hipError_t launch_record(const ExpandArgs& a, uint32_t n, hipStream_t st) {
     if (!n) return hipSuccess;
-    hipLaunchKernelGGL(k_dedup, dim3((n + 255) / 256), dim3(256), 0, st, C, n, runs, ctr);
+    const uint32_t chunk = WAVE * ((n + WAVE * kRecordWaves - 1) / (WAVE * kRecordWaves));
+    const uint32_t waves = (n + chunk - 1) / chunk;
+    hipLaunchKernelGGL(k_record, dim3((waves + 3) / 4), dim3(256), 0, st, a, n, chunk);
     return hipGetLastError();
 }
 
@@ -1630,6 +1730,37 @@ static void launch_expand_team(const ExpandArgs& a, uint32_t grid, uint32_t wpb,
 
 uint32_t expand_grid(uint32_t n_items, uint32_t team, uint32_t wpb, uint32_t grid_cap, uint32_t lanes) {
     return grid_for(n_items, team == 1 ? wpb * (64 / lanes) : 1, grid_cap);
+}
+
+uint32_t expand_small_lds(uint32_t max_child_ne, uint32_t max_nextv, uint32_t A) {
+    return (SmallSizes::make(max_child_ne, max_nextv, A).bytes(A) + 15u) & ~15u;
+}
+
+template <uint32_t UA>
+static hipError_t launch_expand_small_ua(const ExpandArgs& a, uint32_t grid, uint32_t wpb, uint32_t lanes,
+                                         hipStream_t st) {
+    const dim3 g(grid), b(64 * wpb);
+    const size_t lds = (size_t)a.lds_per_wave * wpb * (64 / lanes);
+    switch (lanes) {
+        case 64: hipLaunchKernelGGL((k_expand_small<UA, 64>), g, b, lds, st, a); break;
+        case 32: hipLaunchKernelGGL((k_expand_small<UA, 32>), g, b, lds, st, a); break;
+        case 16: hipLaunchKernelGGL((k_expand_small<UA, 16>), g, b, lds, st, a); break;
+        case 8: hipLaunchKernelGGL((k_expand_small<UA, 8>), g, b, lds, st, a); break;
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_expand_small(const ExpandArgs& a, uint32_t grid_cap, uint32_t wpb, uint32_t lanes, hipStream_t st) {
+    if (!a.n_items) return hipSuccess;
+    if (!a.lean || a.scratch || a.max_child_ne > kSmallMaxEdges || a.max_nextv > kSmallMaxLabels || a.C.A > 4 ||
+        a.M.K > lanes)
+        return hipErrorInvalidValue;
+    ExpandArgs x = a;
+    const uint32_t grid = expand_grid(a.n_items, 1, wpb, grid_cap, lanes);
+    x.chunk = (uint64_t)grid * wpb * (64 / lanes) >= a.n_items ? 1u : 2u;
+    return x.P.A == 2 && a.C.A == 2 ? launch_expand_small_ua<2>(x, grid, wpb, lanes, st)
+                                    : launch_expand_small_ua<0>(x, grid, wpb, lanes, st);
 }
 
 hipError_t launch_expand(const ExpandArgs& a, uint32_t grid_cap, uint32_t wpb, uint32_t team, hipStream_t st,

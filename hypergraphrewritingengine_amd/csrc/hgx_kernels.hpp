@@ -79,15 +79,8 @@ struct ExpandArgs {
     uint32_t nrange;
     uint32_t n_items;          // children this launch covers
     uint32_t lean;             // every child has one arity 2..4 and < 2^16 edges: lean workspace
-    uint16_t* tcnt;            // [M] per child: causal triples | triples kept by TR << 8
+    uint32_t chunk;            // k_expand_small: consecutive children per turn of a team
 };
-
-// One run's children in a generation, for k_run_events.
-struct RunEvents {
-    uint32_t slot, cb, ce;
-};
-hipError_t launch_run_events(const RunEvents* items, uint32_t n, const EventView& E, const uint16_t* tcnt,
-                             uint64_t* ctr, hipStream_t st);
 
 // Workspace of one child in k_expand: the hash's, with room in its nbr region for the
 // label -> local id map and in its srt region for the child's vertex labels.
@@ -190,8 +183,14 @@ uint32_t expand_lds_per_wave(uint32_t max_child_ne, uint32_t max_nv, uint32_t ma
 // (64, or 32 / 16 for sub-wave teams, several small children per wave, LDS workspaces only).
 hipError_t launch_expand(const ExpandArgs& a, uint32_t grid_cap, uint32_t wpb, uint32_t team, hipStream_t st,
                          uint32_t lanes = 64);
+// Small children (every one of one arity 2..4, at most kSmallMaxEdges edges and kSmallMaxLabels vertex
+// labels): workspace bytes per child and the launch; lanes per child 8 (matches of at most 8
+// edges), 16, 32 or 64.
+uint32_t expand_small_lds(uint32_t max_child_ne, uint32_t max_nextv, uint32_t A);
+hipError_t launch_expand_small(const ExpandArgs& a, uint32_t grid_cap, uint32_t wpb, uint32_t lanes, hipStream_t st);
 uint32_t expand_grid(uint32_t n_items, uint32_t team, uint32_t wpb, uint32_t grid_cap, uint32_t lanes = 64);
-hipError_t launch_dedup(const GenView& C, uint32_t n, DRun* runs, uint64_t* ctr, hipStream_t st);
+// Records, identity and counters of the n children of a.M, whose hashes k_expand left in a.C.hash.
+hipError_t launch_record(const ExpandArgs& a, uint32_t n, hipStream_t st);
 // grid used by the launchers for `items` work items (for sizing global scratch)
 uint32_t launch_grid(uint32_t items, uint32_t wpb, uint32_t grid_cap);
 uint32_t branchial_lds_per_wave();
