@@ -230,6 +230,8 @@ constexpr uint32_t kClassEdges[6] = {32, 64, 128, 512, 2048, 0xFFFFFFFFu};
 // up to 32 edges, or two of up to 64, each in its own workspace; the autotuner may choose others).
 constexpr int kExpandClasses = 6;
 constexpr uint32_t kExpandEdges[kExpandClasses] = {32, 64, 128, 512, 2048, 0xFFFFFFFFu};
+constexpr int kMergeClass = 2;               // the largest of the merged classes (up to 128 edges)
+constexpr uint64_t kMergeBelow = 32768;      // states or children
 static_assert(kExpandClasses == kTuneExpandClasses, "one tuned shape per expansion size class");
 static_assert(sizeof(kClassEdges) / sizeof(kClassEdges[0]) == kTuneJoinClasses, "one tuned shape per join size class");
 
@@ -464,13 +466,21 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
             auto launch_classes = [&](bool emit, std::vector<ExpandClass>& cls, const char* name,
                                       uint64_t bytes) {
                 cls.assign(6, ExpandClass{});
+                // few states of up to 128 edges: one class of them all, as for the children
+                uint64_t n_small = 0;
+                for (uint32_t i = 0; i < nF; ++i)
+                    if ((emit ? tot[i] != 0 : h_active[F_runs_[i]->slot] != 0) &&
+                        F_runs_[i]->ne_bound <= kClassEdges[kMergeClass])
+                        n_small += F_e_[i] - F_b_[i];
+                const bool merge = n_small < kMergeBelow;
                 for (uint32_t i = 0; i < nF; ++i) {
                     const RunRec& r = *F_runs_[i];
                     if (emit ? !tot[i] : !h_active[r.slot]) continue;
                     if (F_e_[i] == F_b_[i]) continue;
                     int k = 0;
                     while (r.ne_bound > kClassEdges[k]) ++k;
-                        ExpandClass& x = cls[k];
+                    if (merge && k < kMergeClass) k = kMergeClass;
+                    ExpandClass& x = cls[k];
                     x.ne = std::max(x.ne, r.ne_bound);
                     x.nextv = std::max(x.nextv, r.nv_bound);
                     x.rb.push_back(F_b_[i]);
@@ -808,12 +818,22 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
             // Size classes: children grouped by their request's bound on child edges, each class
             // launched with a workspace sized for it, so one large request in the mix does not
             // push every child onto the large-state workspace.
+            // Children of up to 128 edges in a generation of few children are one class: a launch
+            // of a few thousand children lasts as long as its slowest, so one launch of them
+            // all is shorter than one after another (61 requests, joins and expansion merged:
+            // 2.62 -> 2.04 ms; the same with the line at 8,192, 2.17, or 131,072, 2.06).
+            uint64_t n_small = 0;
+            for (uint32_t i = 0; i < nF; ++i)
+                if (tot[i] && F_runs_[i]->ne_bound + F_runs_[i]->hp->max_gain <= kExpandEdges[kMergeClass])
+                    n_small += tot[i];
+            const bool merge = n_small < kMergeBelow;
             for (uint32_t i = 0; i < nF; ++i) {
                 if (!tot[i]) continue;
                 const RunRec& r = *F_runs_[i];
                 const uint32_t cne = r.ne_bound + r.hp->max_gain, cnv = r.nv_bound + r.hp->max_new;
                 int k = 0;
                 while (cne > kExpandEdges[k]) ++k;
+                if (merge && k < kMergeClass) k = kMergeClass;
                 ExpandClass& x = cls[k];
                 x.ne = std::max(x.ne, cne);
                 x.nextv = std::max(x.nextv, cnv);
