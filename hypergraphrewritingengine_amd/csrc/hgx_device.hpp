@@ -57,6 +57,13 @@ struct DRule {
     // remaining positions greedily by shared variables; apiv[p] are its pivots.
     uint8_t aord[16][16];
     uint8_t apiv[16][16];
+    // The join over binary edges by bit sets (k_match_bits), for rules of at most 4 LHS edges, all
+    // binary (bits_ok): per join depth, where the variable of each position was bound -- for
+    // position 0 bit 0 set when it was, bits 1-2 the depth, bit 3 the position there; the same in
+    // bits 4-7 for position 1; bit 8: position 1 repeats position 0 -- and in bits 12-13 the LHS
+    // index of the pattern edge.
+    uint32_t bits_ok, pad2[3];
+    uint32_t bj[4];
 };
 static_assert(offsetof(DRule, lv) % 4 == 0 && sizeof(DRule) % 4 == 0, "DRule is staged in 32-bit words");
 

@@ -2,6 +2,7 @@
 //
 //   k_match<false>   SCAN -> EXPAND -> SINK join, counting matches per state
 //   k_match<true>    the same join, writing match records in the deterministic order
+//   k_match_bits     both over small binary states, by bit sets
 //   k_expand         rewrite + WL hash, one team per child state
 //                    (k_expand_small: small children of one arity)
 //   k_record         each child's event, causal masks and records, its hash into its request's
@@ -344,6 +345,8 @@ uint32_t match_lds_per_wave(uint32_t max_ne, uint32_t max_nextv, uint32_t A, uin
     return b;
 }
 
+constexpr uint64_t kNoBudget = 0xFFFFFFFFull;    // MatchArgs::budget of a run without a cap
+
 // W is the team: one wave per state (W = 1, up to four per workgroup, each with its own
 // workspace) or the W waves of a workgroup sharing one state and one workspace (large states,
 // whose workspace would otherwise leave a CU one or two waves). The one-wave passes are held to
@@ -424,8 +427,10 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W, W == 1 ? 4 : 1) void k_match
         const uint32_t nvid = a.P.nextv[s];                     // labels are < nvid
         const uint8_t active = a.active[run] && (!a.smask || a.smask[s]);
         const uint64_t budget = EMIT ? 0 : (uint64_t)a.budget[run];
-        // the run's tally moves under other teams: one read, shared, so the team agrees
-        const uint64_t tally = EMIT ? 0 : tm.bcast(tm.leader() ? (uint64_t)a.run_acc[run] : 0ull);
+        // the run's tally moves under other teams: one read, shared, so the team agrees. A run without
+        // a cap keeps none: the adds of one run's 300 k states to one word took 4 ms.
+        const bool capped = !EMIT && budget != kNoBudget;
+        const uint64_t tally = capped ? tm.bcast(tm.leader() ? (uint64_t)a.run_acc[run] : 0ull) : 0ull;
         if (!active || (!EMIT && tally > budget)) {
             if (!EMIT && tm.leader()) { a.cnt[s] = 0; a.state_edges[s] = 0; }
             continue;
@@ -617,7 +622,7 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W, W == 1 ? 4 : 1) void k_match
                 } else {
                     total = nf + nd;
                     edges_sum = tm.sum64(de);
-                    if (tm.leader() && total) atomicAdd(&a.run_acc[run], (unsigned long long)total);
+                    if (tm.leader() && total && capped) atomicAdd(&a.run_acc[run], (unsigned long long)total);
                 }
             }
         }
@@ -686,7 +691,8 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W, W == 1 ? 4 : 1) void k_match
                     const uint32_t round = tm.sum(c);
                     total += round;
                     edges_sum += (uint64_t)round * child_ne;
-                    if (base + N >= nseed && r + 1 >= RN.n_rules) {
+                    if (!capped) {
+                    } else if (base + N >= nseed && r + 1 >= RN.n_rules) {
                         // the state's last round: nothing is left to stop, so add without waiting
                         if (tm.leader() && round) atomicAdd(&a.run_acc[run], (unsigned long long)round);
                     } else {
@@ -706,6 +712,273 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W, W == 1 ? 4 : 1) void k_match
     }
 }
 
+
+// ------------------------------------------------------------------------------------------
+// The join over small binary states by bit sets: states of at most 64 * NW edges and 255 vertex labels,
+// every edge binary, rules of at most 4 LHS edges. Per (position, vertex) a set of the edges holding
+// the vertex there, one bit an edge, in LDS; the candidates of a depth are the intersection of the
+// sets of its bound positions (and the loops where the pattern edge repeats its variable) less the
+// edges in use, so no candidate is tested, the ascending order is the bits', and the last depth
+// counts by population count. Matches and their order are k_match's. What bounded k_match here were
+// chains of LDS reads per candidate -- list entry, edge, rule tables; this one is bound by the state's
+// loads and the building of the sets (batched pass: count 4.10 -> 0.85 ms, emit 1.80 -> 0.36).
+// ------------------------------------------------------------------------------------------
+
+template <uint32_t NW>
+struct BitSet {
+    uint64_t w[NW];
+};
+
+template <uint32_t NW>
+struct BitJoin {
+    const uint64_t* inc0;      // [labels][NW]
+    const uint64_t* inc1;
+    const uint16_t* ev;        // edges: first vertex | second << 8
+    BitSet<NW> all, loops;
+    uint32_t bj[4];
+};
+
+// The edges bound so far and their vertices, by value and by constant depth: registers.
+struct Bound {
+    uint32_t e0, e1, e2, e3, v0, v1, v2, v3;
+    template <int D>
+    __device__ __forceinline__ void set(uint32_t x, uint32_t v) {
+        if constexpr (D == 1) { e1 = x; v1 = v; }
+        else if constexpr (D == 2) { e2 = x; v2 = v; }
+        else { e3 = x; v3 = v; }
+    }
+};
+
+// Candidates of depth D, whose binding word is b.
+template <uint32_t NW, int D>
+__device__ __forceinline__ BitSet<NW> bit_cands(const BitJoin<NW>& J, uint32_t b, const Bound& B) {
+    auto value = [&](uint32_t src) {                 // a bound position's vertex
+        const uint32_t d = (src >> 1) & 3u;
+        uint32_t x = B.v0;
+        // (masks, not selects: a select of two members makes the struct live in memory)
+        if (D > 1) { const uint32_t m = 0u - (uint32_t)(d == 1); x = (x & ~m) | (B.v1 & m); }
+        if (D > 2) { const uint32_t m = 0u - (uint32_t)(d == 2); x = (x & ~m) | (B.v2 & m); }
+        return (src & 8u) ? x >> 8 : x & 0xFFu;
+    };
+    BitSet<NW> m = J.all;
+    if (b & 1u) {
+        const uint64_t* s = J.inc0 + value(b) * NW;
+#pragma unroll
+        for (uint32_t k = 0; k < NW; ++k) m.w[k] &= s[k];
+    }
+    if (b & 16u) {
+        const uint64_t* s = J.inc1 + value(b >> 4) * NW;
+#pragma unroll
+        for (uint32_t k = 0; k < NW; ++k) m.w[k] &= s[k];
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < NW; ++k) {
+        if (b & 256u) m.w[k] &= J.loops.w[k];
+        auto drop = [&](uint32_t e) { if (NW == 1 || (e >> 6) == k) m.w[k] &= ~(1ull << (e & 63u)); };
+        drop(B.e0);
+        if (D > 1) drop(B.e1);
+        if (D > 2) drop(B.e2);
+    }
+    return m;
+}
+
+// Completions of depths D..N-1; OUT writes each as the found-th match of `o`, else counts.
+template <uint32_t NW, int N, int D, bool OUT>
+__device__ __forceinline__ uint32_t bit_join(const BitJoin<NW>& J, Bound B, const RegJoinOut& o, uint32_t found) {
+    if constexpr (D == N) {
+        if constexpr (OUT) {
+            const size_t at = (size_t)(o.base + found);
+            if (N == 2 && o.K == 2) {                 // the pair in one word
+                const bool swap = ((J.bj[0] >> 12) & 3u) != 0;
+                ((uint32_t*)o.q)[at] = swap ? (B.e1 | B.e0 << 16) : (B.e0 | B.e1 << 16);
+            } else {
+                uint16_t* q = o.q + at * o.K;
+                q[(J.bj[0] >> 12) & 3u] = (uint16_t)B.e0;
+                if (N > 1) q[(J.bj[1] >> 12) & 3u] = (uint16_t)B.e1;
+                if (N > 2) q[(J.bj[2] >> 12) & 3u] = (uint16_t)B.e2;
+                if (N > 3) q[(J.bj[3] >> 12) & 3u] = (uint16_t)B.e3;
+            }
+            o.parent[at] = o.state; o.rule[at] = o.rule_id; o.cne[at] = o.child_ne;
+        }
+        return found + 1;
+    } else {
+        const BitSet<NW> m = bit_cands<NW, D>(J, J.bj[D], B);
+#pragma unroll
+        for (uint32_t k = 0; k < NW; ++k) {
+            if constexpr (D + 1 == N && !OUT) {
+                found += (uint32_t)__popcll(m.w[k]);
+            } else {
+                for (uint64_t w = m.w[k]; w; w &= w - 1) {
+                    const uint32_t e = k * 64 + (uint32_t)__builtin_ctzll(w);
+                    B.template set<D>(e, D + 1 < N ? J.ev[e] : 0u);
+                    found = bit_join<NW, N, D + 1, OUT>(J, B, o, found);
+                }
+            }
+        }
+        return found;
+    }
+}
+
+template <uint32_t NW, bool OUT>
+__device__ __forceinline__ uint32_t bit_join_any(const BitJoin<NW>& J, uint32_t n_lhs, uint32_t seed, uint32_t sv,
+                                                 const RegJoinOut& o) {
+    const Bound B{seed, 0, 0, 0, sv, 0, 0, 0};
+    switch (n_lhs) {
+        case 1: return bit_join<NW, 1, 1, OUT>(J, B, o, 0u);
+        case 2: return bit_join<NW, 2, 1, OUT>(J, B, o, 0u);
+        case 3: return bit_join<NW, 3, 1, OUT>(J, B, o, 0u);
+        default: return bit_join<NW, 4, 1, OUT>(J, B, o, 0u);
+    }
+}
+
+uint32_t match_bits_lds(uint32_t max_ne, uint32_t max_nextv, uint32_t nw) {
+    return (2 * max_nextv * nw * 8 + ((2 * max_ne + 7u) & ~7u) + 15u) & ~15u;
+}
+
+template <bool EMIT, uint32_t NW, uint32_t G>
+__global__ __launch_bounds__(256) void k_match_bits(MatchArgs a) {
+    using TM = typename TeamSel<1, G>::type;
+    extern __shared__ uint8_t lds[];
+    constexpr uint32_t N = TM::N;
+    const uint32_t tpb = (blockDim.x / WAVE) * (WAVE / G), ti = threadIdx.x / G;
+    uint8_t* p = lds + (size_t)ti * a.lds_per_wave;
+    const TM tm(nullptr);
+    const uint32_t A = a.P.A, NL = a.max_nextv;
+    uint64_t* inc0 = (uint64_t*)carve(p, NL * NW * 8);
+    uint64_t* inc1 = (uint64_t*)carve(p, NL * NW * 8);
+    uint16_t* ev = (uint16_t*)carve(p, a.max_ne * 2);
+
+    // states strided over the teams, the count pass's scattered in blocks, as in k_match
+    const uint32_t teams = gridDim.x * tpb;
+    const uint32_t n_items = a.nrange ? a.n_items : a.P.n;
+    const bool spread = !EMIT && a.spread > 1;
+    const uint32_t nblk = (n_items + kCountSpreadBlock - 1) / kCountSpreadBlock;
+    const uint32_t n_loop = spread ? nblk * kCountSpreadBlock : n_items;
+    for (uint32_t ls = blockIdx.x * tpb + ti; ls < n_loop; ls += teams) {
+        uint32_t s = ls;
+        if (spread) {
+            s = (uint32_t)((uint64_t)(ls / kCountSpreadBlock) * a.spread % nblk) * kCountSpreadBlock +
+                ls % kCountSpreadBlock;
+            if (s >= n_items) continue;                         // the last block's tail
+        }
+        if (a.nrange) {                                         // subset: logical -> state
+            uint32_t lo = 0, hi = a.nrange;
+            while (hi - lo > 1) { const uint32_t mid = (lo + hi) >> 1; if (a.rpre[mid] <= s) lo = mid; else hi = mid; }
+            s = a.rb[lo] + (s - a.rpre[lo]);
+        }
+        const uint32_t run = a.P.run[s];
+        const uint32_t ne = a.P.ne[s];
+        const uint64_t eo = a.P.eoff[s];
+        const uint32_t nvid = a.P.nextv[s];                     // labels are < nvid
+        const uint32_t nm = EMIT ? a.cnt[s] : 0u;
+        const uint8_t active = a.active[run] && (!a.smask || a.smask[s]);
+        const uint64_t budget = EMIT ? 0 : (uint64_t)a.budget[run];
+        const bool capped = !EMIT && budget != kNoBudget;
+        const uint64_t tally = capped ? tm.bcast(tm.leader() ? (uint64_t)a.run_acc[run] : 0ull) : 0ull;
+        if (!active || (EMIT ? nm == 0 : tally > budget)) {
+            if (!EMIT && tm.leader()) { a.cnt[s] = 0; a.state_edges[s] = 0; }
+            continue;
+        }
+        const DRun& RN = a.runs[run];
+        const DRule* rules = RN.rules;
+        const uint32_t n_rules = RN.n_rules;
+        tm.sync();
+        for (uint32_t i = tm.r; i < nvid * NW; i += N) { inc0[i] = 0; inc1[i] = 0; }
+        tm.sync();
+        BitJoin<NW> J;
+        J.inc0 = inc0; J.inc1 = inc1; J.ev = ev;
+#pragma unroll
+        for (uint32_t k = 0; k < NW; ++k) {
+            J.loops.w[k] = 0;
+            J.all.w[k] = ne >= 64 * (k + 1) ? ~0ull : ne > 64 * k ? (1ull << (ne - 64 * k)) - 1ull : 0ull;
+        }
+        for (uint32_t base = 0; base < ne; base += N) {
+            const uint32_t e = base + tm.r;
+            uint32_t x = 0, y = 1;
+            if (e < ne) {
+                if (A == 2) { const uint2 v = ((const uint2*)a.P.ev)[eo + e]; x = v.x; y = v.y; }
+                else { x = a.P.ev[(eo + e) * A]; y = a.P.ev[(eo + e) * A + 1]; }
+                ev[e] = (uint16_t)(x | y << 8);
+                atomicOr((unsigned long long*)&inc0[x * NW + (e >> 6)], 1ull << (e & 63u));
+                atomicOr((unsigned long long*)&inc1[y * NW + (e >> 6)], 1ull << (e & 63u));
+            }
+            const uint64_t lb = tm.ballot(e < ne && x == y) << (base & 63u);
+#pragma unroll
+            for (uint32_t k = 0; k < NW; ++k)
+                if ((base >> 6) == k) J.loops.w[k] |= lb;
+        }
+        tm.sync();
+        uint32_t total = 0;
+        uint64_t edges_sum = 0;                                // count pass: edges of the children
+        uint32_t out = EMIT ? (uint32_t)a.moff[s] : 0u;
+        for (uint32_t r = 0; r < n_rules; ++r) {
+            const DRule& R = rules[r];
+            if (!R.bits_ok) continue;                           // a pattern edge that is not binary
+            const uint32_t n_lhs = R.n_lhs, child_ne = ne - n_lhs + R.n_rhs;
+#pragma unroll
+            for (int d = 0; d < 4; ++d) J.bj[d] = R.bj[d];
+            uint32_t mine = 0;
+            for (uint32_t base = 0; base < ne; base += N) {
+                const uint32_t seed = base + tm.r;
+                const uint32_t sv = seed < ne ? ev[seed] : 0u;
+                const bool ok = seed < ne && (!(J.bj[0] & 256u) || (sv & 0xFFu) == sv >> 8);
+                const uint32_t c = ok ? bit_join_any<NW, false>(J, n_lhs, seed, sv, RegJoinOut{}) : 0u;
+                mine += c;
+                if constexpr (EMIT) {
+                    uint32_t round;
+                    const uint32_t inc = tm.incl_scan(c, round);
+                    if (c) {
+                        const RegJoinOut ro{a.M.q, a.M.K, out + inc - c, a.M.parent, a.M.rule, a.M.cne, s, r, child_ne};
+                        bit_join_any<NW, true>(J, n_lhs, seed, sv, ro);
+                    }
+                    out += round;
+                }
+            }
+            if constexpr (!EMIT) {
+                const uint32_t sum = tm.sum(mine);
+                total += sum;
+                edges_sum += (uint64_t)sum * child_ne;
+            }
+        }
+        if (!EMIT && tm.leader()) {
+            a.cnt[s] = total;
+            a.state_edges[s] = edges_sum;
+            // the run's shared tally: past what the run may still take its other states are skipped
+            if (total && capped) atomicAdd(&a.run_acc[run], (unsigned long long)total);
+        }
+    }
+}
+
+template <uint32_t NW>
+static hipError_t launch_match_bits_nw(const MatchArgs& a, bool emit, uint32_t grid, uint32_t wpb, uint32_t lanes,
+                                       hipStream_t st) {
+    const dim3 g(grid), b(64 * wpb);
+    const size_t lds = (size_t)a.lds_per_wave * wpb * (64 / lanes);
+    switch (lanes + (emit ? 1 : 0)) {
+        case 16: hipLaunchKernelGGL((k_match_bits<false, NW, 16>), g, b, lds, st, a); break;
+        case 17: hipLaunchKernelGGL((k_match_bits<true, NW, 16>), g, b, lds, st, a); break;
+        case 32: hipLaunchKernelGGL((k_match_bits<false, NW, 32>), g, b, lds, st, a); break;
+        case 33: hipLaunchKernelGGL((k_match_bits<true, NW, 32>), g, b, lds, st, a); break;
+        case 64: hipLaunchKernelGGL((k_match_bits<false, NW, 64>), g, b, lds, st, a); break;
+        case 65: hipLaunchKernelGGL((k_match_bits<true, NW, 64>), g, b, lds, st, a); break;
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+uint32_t launch_grid(uint32_t items, uint32_t wpb, uint32_t grid_cap);
+
+hipError_t launch_match_bits(const MatchArgs& a, bool emit, uint32_t grid_cap, uint32_t wpb, hipStream_t st,
+                             uint32_t lanes) {
+    const uint32_t items = a.nrange ? a.n_items : a.P.n;
+    if (!items) return hipSuccess;
+    const uint32_t nw = match_bits_words(a.max_ne);
+    if (!nw || a.max_nextv > kMatchBitsLabels || a.scratch || a.fwd_n || a.P.A < 2) return hipErrorInvalidValue;
+    const uint32_t grid = launch_grid(items, wpb * (64 / lanes), grid_cap);
+    return nw == 1 ? launch_match_bits_nw<1>(a, emit, grid, wpb, lanes, st)
+           : nw == 2 ? launch_match_bits_nw<2>(a, emit, grid, wpb, lanes, st)
+                     : launch_match_bits_nw<4>(a, emit, grid, wpb, lanes, st);
+}
 
 // ------------------------------------------------------------------------------------------
 // Rewrite + hash, one team per child, then the children's records (Rewriter::apply,

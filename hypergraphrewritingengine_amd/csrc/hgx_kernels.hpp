@@ -177,6 +177,14 @@ hipError_t launch_copy_roots(const RootCopy* items, uint32_t n, const GenView& v
 // states per wave, each with its own lds_per_wave workspace), 64 for one wave per state.
 hipError_t launch_match(const MatchArgs& a, bool emit, uint32_t grid_cap, uint32_t wpb, uint32_t team,
                         hipStream_t st, uint32_t lanes = 64);
+// Small binary states (every edge binary, at most 255 edges and labels, no forwarding, rules of at most
+// 4 LHS edges): 64-bit words per edge set, 0 when a state can be too large; workspace bytes per state
+// and the launch, lanes per state 16, 32 or 64.
+constexpr uint32_t kMatchBitsLabels = 255;
+inline uint32_t match_bits_words(uint32_t max_ne) { return max_ne <= 64 ? 1 : max_ne <= 128 ? 2 : max_ne <= 255 ? 4 : 0; }
+uint32_t match_bits_lds(uint32_t max_ne, uint32_t max_nextv, uint32_t nw);
+hipError_t launch_match_bits(const MatchArgs& a, bool emit, uint32_t grid_cap, uint32_t wpb, hipStream_t st,
+                             uint32_t lanes);
 uint32_t expand_lds_per_wave(uint32_t max_child_ne, uint32_t max_nv, uint32_t max_nextv, uint32_t A, bool lean);
 // team: waves per child (1, 2, 4 or 8); with team 1, wpb children per workgroup.
 // team: waves sharing one child (1, 2, 4, 8); lanes: with team 1, the lanes sharing one child

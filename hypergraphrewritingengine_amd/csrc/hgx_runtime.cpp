@@ -285,6 +285,18 @@ void parse_rules(const uint8_t* p, uint32_t len, uint32_t n, std::vector<DRule>&
                 }
             }
         }
+        R.bits_ok = R.n_lhs <= 4 ? 1u : 0u;
+        for (int d = 0; d < R.n_lhs; ++d) R.bits_ok &= R.la[d] == 2 ? 1u : 0u;
+        for (int d = 0; R.bits_ok && d < R.n_lhs; ++d) {
+            uint32_t w = (uint32_t)R.order[d] << 12;
+            for (int i = 0; i < 2; ++i) {
+                const uint32_t src = R.jsrc[d][i];
+                if (src == 0xFF) continue;
+                if ((int)(src >> 4) == d) w |= 1u << 8;
+                else w |= (1u | (src >> 4) << 1 | (src & 1u) << 3) << (4 * i);
+            }
+            R.bj[d] = w;
+        }
         // anchored orders: position p first, then most shared bound variables (ties: lower
         // position); the choice only affects join cost, never the set of matches
         std::memset(R.aord, 0, sizeof(R.aord));
@@ -410,6 +422,8 @@ RunHost parse_run(const hgx_run_desc* d, bool evolve) {
     for (auto& R : h.rules)
         for (int e = 0; e < R.n_rhs; ++e) { amin = std::min<uint32_t>(amin, R.ra[e]); amax = std::max<uint32_t>(amax, R.ra[e]); }
     h.uni_arity = (amin == amax && amax >= 2 && amax <= 4) ? amax : 0u;
+    h.bits_join = h.uni_arity == 2;
+    for (auto& R : h.rules) h.bits_join = h.bits_join && R.n_lhs <= 4;
     // edge positions (match list) and local vertex ids (hash workspaces) are 16-bit: refused
     // before any kernel sees a state that could exceed them (one larger state's matches:
     // hgx_match_count)

@@ -227,6 +227,7 @@ struct RunHost {
     uint32_t max_arity = 1, max_lhs = 1, max_gain = 0, max_new = 0;
     uint32_t uni_arity = 0;      // k when every root edge and every RHS edge has arity k (2..4),
                                  // so every state of the run does; else 0
+    bool bits_join = false;      // binary edges only and rules of at most 4 LHS edges (k_match_bits)
     bool root_uni = false;       // every root edge has one arity 2..4 (the roots alone)
     uint64_t root_edges = 0;
     // quotient exploration: only the first state of each exact class is expanded
