@@ -155,6 +155,7 @@ __device__ __forceinline__ uint64_t dpp(uint64_t v) {
 constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E;               // quad permutations [1,0,3,2], [2,3,0,1]
 constexpr int kDppHalfMirror = 0x141, kDppMirror = 0x140;     // lane i <-> 7 - i, i <-> 15 - i
 constexpr int kDppRowShr = 0x110;                             // + n: from the lane n below in the row
+constexpr int kDppRowShl = 0x100, kDppRowRor = 0x120;         // + n: from the lane n above; from n below, rotating
 constexpr int kDppBcast15 = 0x142, kDppBcast31 = 0x143;       // a row's / half's last lane to the next
 
 // v of the other row of the pair (H = 16) or of the other half of the wave (H = 32): the swap of a

@@ -26,6 +26,7 @@
 #include "hgx_kernels.hpp"
 #include "hgx_wl.hpp"
 #include "hgx_wl_small.hpp"
+#include "hgx_wl_large.hpp"
 
 namespace hgx {
 
@@ -1004,6 +1005,19 @@ __device__ inline bool map_insert(DRun* run, uint64_t h) {
     }
 }
 
+// The hash h of given state i: stored and, for a root, inserted into its run's state map.
+__device__ inline void wl_state_done(const WLStatesArgs& a, uint32_t i, uint64_t h) {
+    a.out[i] = h;
+    if (a.run_of) {
+        DRun* RN = &a.runs[a.run_of[i]];
+        if (map_insert(RN, h)) {
+            atomicAdd((unsigned long long*)&a.ctr[(size_t)a.run_of[i] * CTR_N + CTR_CANON], 1ull);
+            atomicAdd((unsigned long long*)&a.ctr[(size_t)a.run_of[i] * CTR_N + CTR_FINGERPRINT],
+                      (unsigned long long)mix64(h));
+        }
+    }
+}
+
 // GWS selects the workspace at compile time (global scratch for states too large for LDS), so
 // the LDS variant addresses its workspace with LDS instructions rather than flat ones. W is the
 // team: W = 1, one wave per child (up to four per workgroup, each with its own workspace);
@@ -1240,6 +1254,139 @@ __global__ __launch_bounds__(256, 5) void k_expand_small(ExpandArgs a) {
         const uint64_t h = wl_hash_small<UA>(s, tm, cne, nextv, ua);
         if (tm.leader()) a.C.hash[c] = h;              // the child's other records: k_record
         tm.sync();
+    }
+}
+
+// k_expand for large children of one arity (past k_expand_small's limits, within hgx_wl_large.hpp's): the
+// W waves of a workgroup rewrite one child and hash it with its colours in LDS. ALL: every array of the
+// hash in LDS, else the ones walked in order in a slice of a.scratch per workgroup.
+template <uint32_t UA, uint32_t W, bool ALL>
+__global__ __launch_bounds__(64 * W) void k_expand_large(ExpandArgs a) {
+    extern __shared__ uint8_t lds[];
+    const uint32_t PA = UA ? UA : a.P.A, A = UA ? UA : a.C.A;              // parent / child vertex strides
+    const LargeSizes z = LargeSizes::make(a.max_child_ne, a.max_nextv, A);
+    LargeSpace s;
+    large_bind<ALL>(s, lds, ALL ? nullptr : a.scratch + (size_t)blockIdx.x * z.rest(), z);
+    const Team<W> tm(s.red);
+    const uint32_t l = tm.r;
+    for (uint32_t lc = xcd_block(); lc < a.n_items; lc += gridDim.x) {
+        uint32_t c = lc;
+        if (a.nrange) {
+            uint32_t lo = 0, hi = a.nrange;
+            while (hi - lo > 1) { const uint32_t mid = (lo + hi) >> 1; if (a.rpre[mid] <= lc) lo = mid; else hi = mid; }
+            c = a.rb[lo] + (lc - a.rpre[lo]);
+        }
+        const uint32_t par = a.M.parent[c];
+        const uint64_t ceo = a.C.eoff[c];
+        const uint32_t run = a.P.run[par];
+        const uint32_t pne = a.P.ne[par];
+        const uint64_t peo = a.P.eoff[par];
+        const uint32_t fresh_base = a.P.nextv[par];
+        const DRule& R = a.runs[run].rules[a.M.rule[c]];
+        const uint32_t nl = R.n_lhs, nr = R.n_rhs;
+        const uint32_t ua = UA ? UA : R.la[0];
+        const uint32_t cne = pne - nl + nr, kept = pne - nl;
+        if (l < nl) s.q[l] = a.M.q[(size_t)c * a.M.K + l];
+        tm.sync();
+        // parent edges minus the consumed ones, order kept (SparseBitset::derive)
+        for (uint32_t i = l; i < pne; i += 64 * W) {
+            bool keep = true;
+            uint32_t pos = i;
+            for (uint32_t t = 0; t < nl; ++t) {
+                const uint32_t q = s.q[t];
+                keep &= q != i;
+                pos -= q < i ? 1u : 0u;
+            }
+            if (!keep) continue;
+            if constexpr (UA == 2) {
+                ((uint2*)a.C.ev)[ceo + pos] = ((const uint2*)a.P.ev)[peo + i];
+            } else {
+                for (uint32_t k = 0; k < A; ++k) a.C.ev[(ceo + pos) * A + k] = k < PA ? a.P.ev[(peo + i) * PA + k] : 0u;
+            }
+            a.C.ar[ceo + pos] = (uint8_t)ua;
+            a.C.ps[ceo + pos] = a.P.ps[peo + i];
+        }
+        // produced edges in RHS order; fresh vertices ascending by variable
+        // (assign_fresh_consecutive / resolve_rhs_vertices, rewrite_core.hpp:53-87)
+        if (l < nr) {
+            const uint32_t pos = kept + l;
+            for (uint32_t k = 0; k < A; ++k) {
+                uint32_t v = 0;
+                if (k < ua) {
+                    const uint32_t var = R.rv[l][k];
+                    if (R.lhs_mask & (1u << var)) v = a.P.ev[(peo + s.q[R.var_src_edge[var]]) * PA + R.var_src_pos[var]];
+                    else v = fresh_base + __popc(R.new_mask & ((1u << var) - 1u));
+                }
+                a.C.ev[(ceo + pos) * A + k] = v;
+            }
+            a.C.ar[ceo + pos] = (uint8_t)ua;
+            a.C.ps[ceo + pos] = (uint8_t)(a.P.depth[par] + 1u);
+        }
+        tm.sync();
+        const uint64_t h = wl_hash_large<UA, ALL>(s, tm, a.C.ev + ceo * A, A, cne, fresh_base + R.n_new, ua);
+        if (tm.leader()) a.C.hash[c] = h;              // the child's other records: k_record
+        tm.sync();
+    }
+}
+
+// The hash of given states of one arity each, within the same limits.
+template <uint32_t UA, uint32_t W, bool ALL>
+__global__ __launch_bounds__(64 * W) void k_wl_large(WLStatesArgs a) {
+    extern __shared__ uint8_t lds[];
+    const uint32_t A = UA ? UA : a.A;
+    const LargeSizes z = LargeSizes::make(a.max_ne, a.max_nv, A);
+    LargeSpace s;
+    large_bind<ALL>(s, lds, ALL ? nullptr : a.scratch + (size_t)blockIdx.x * z.rest(), z);
+    const Team<W> tm(s.red);
+    for (uint32_t i = blockIdx.x; i < a.n; i += gridDim.x) {
+        const uint64_t e0 = a.state_off[i];
+        const uint32_t ne = (uint32_t)(a.state_off[i + 1] - e0);
+        tm.sync();
+        const uint64_t h = wl_hash_large<UA, ALL>(s, tm, a.ev + e0 * A, A, ne, a.nv[i], UA ? UA : ne ? a.ar[e0] : 2u);
+        if (tm.leader()) wl_state_done(a, i, h);
+    }
+}
+
+uint32_t large_lds(uint32_t max_ne, uint32_t max_nextv, uint32_t A, bool all) {
+    const LargeSizes z = LargeSizes::make(max_ne, max_nextv, A);
+    return (z.hot() + (all ? z.rest() : 0u) + 15u) & ~15u;
+}
+uint32_t large_scratch(uint32_t max_ne, uint32_t max_nextv, uint32_t A) { return LargeSizes::make(max_ne, max_nextv, A).rest(); }
+
+template <uint32_t UA, uint32_t W>
+static hipError_t launch_expand_large_w(const ExpandArgs& a, uint32_t grid, hipStream_t st) {
+    if (a.scratch) hipLaunchKernelGGL((k_expand_large<UA, W, false>), dim3(grid), dim3(64 * W), a.lds_per_wave, st, a);
+    else hipLaunchKernelGGL((k_expand_large<UA, W, true>), dim3(grid), dim3(64 * W), a.lds_per_wave, st, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_expand_large(const ExpandArgs& a, uint32_t grid, uint32_t team, hipStream_t st) {
+    if (!a.n_items) return hipSuccess;
+    if (!a.lean || a.C.A > 4 || !large_fits(a.max_child_ne, a.max_nextv, a.C.A)) return hipErrorInvalidValue;
+    const bool two = a.P.A == 2 && a.C.A == 2;
+    switch (team) {
+        case 4: return two ? launch_expand_large_w<2, 4>(a, grid, st) : launch_expand_large_w<0, 4>(a, grid, st);
+        case 8: return two ? launch_expand_large_w<2, 8>(a, grid, st) : launch_expand_large_w<0, 8>(a, grid, st);
+        case 16: return two ? launch_expand_large_w<2, 16>(a, grid, st) : launch_expand_large_w<0, 16>(a, grid, st);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+template <uint32_t UA, uint32_t W>
+static hipError_t launch_wl_large_w(const WLStatesArgs& a, uint32_t grid, hipStream_t st) {
+    if (a.scratch) hipLaunchKernelGGL((k_wl_large<UA, W, false>), dim3(grid), dim3(64 * W), a.lds_per_wave, st, a);
+    else hipLaunchKernelGGL((k_wl_large<UA, W, true>), dim3(grid), dim3(64 * W), a.lds_per_wave, st, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_wl_large(const WLStatesArgs& a, uint32_t grid, uint32_t team, hipStream_t st) {
+    if (!a.n) return hipSuccess;
+    if (!a.lean || a.A > 4 || !large_fits(a.max_ne, a.max_nv, a.A)) return hipErrorInvalidValue;
+    switch (team) {
+        case 4: return a.A == 2 ? launch_wl_large_w<2, 4>(a, grid, st) : launch_wl_large_w<0, 4>(a, grid, st);
+        case 8: return a.A == 2 ? launch_wl_large_w<2, 8>(a, grid, st) : launch_wl_large_w<0, 8>(a, grid, st);
+        case 16: return a.A == 2 ? launch_wl_large_w<2, 16>(a, grid, st) : launch_wl_large_w<0, 16>(a, grid, st);
+        default: return hipErrorInvalidValue;
     }
 }
 
@@ -1822,17 +1969,7 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W) void k_wl_states(WLStatesArg
         s.nV = a.nv[i];
         tm.sync();
         const uint64_t h = wl_hash_team(s, tm);
-        if (tm.leader()) {
-            a.out[i] = h;
-            if (a.run_of) {
-                DRun* RN = &a.runs[a.run_of[i]];
-                if (map_insert(RN, h)) {
-                    atomicAdd((unsigned long long*)&a.ctr[(size_t)a.run_of[i] * CTR_N + CTR_CANON], 1ull);
-                    atomicAdd((unsigned long long*)&a.ctr[(size_t)a.run_of[i] * CTR_N + CTR_FINGERPRINT],
-                              (unsigned long long)mix64(h));
-                }
-            }
-        }
+        if (tm.leader()) wl_state_done(a, i, h);
         tm.sync();
     }
 }
@@ -2125,6 +2262,7 @@ uint32_t wl_states_grid(uint32_t n, uint32_t team, uint32_t wpb, uint32_t grid_c
 
 hipError_t launch_wl_states(const WLStatesArgs& a, uint32_t grid_cap, uint32_t wpb, uint32_t team, hipStream_t st) {
     if (!a.n) return hipSuccess;
+    if (a.large) return launch_wl_large(a, a.large, team, st);
     const uint32_t grid = wl_states_grid(a.n, team, wpb, grid_cap);
     switch (team) {
         case 1: launch_wl_states_team<1>(a, grid, wpb, st); break;

@@ -6,6 +6,7 @@
 
 #include "hgx_device.hpp"
 #include "hgx_wl.hpp"
+#include "hgx_wl_large.hpp"
 
 namespace hgx {
 
@@ -144,6 +145,7 @@ struct WLStatesArgs {
     uint32_t lds_per_wave;
     uint8_t* scratch;          // as ExpandArgs::scratch
     uint32_t lean;             // every state has one arity 2..4 and < 2^16 edges: lean workspace
+    uint32_t large;            // workgroups of the large-state launch (launch_wl_large); 0: k_wl_states
 };
 
 // lanes: the launch may forward (fwd_n != 0), so the small-rule path needs its per-lane LDS
@@ -196,6 +198,16 @@ hipError_t launch_expand(const ExpandArgs& a, uint32_t grid_cap, uint32_t wpb, u
 // edges), 16, 32 or 64.
 uint32_t expand_small_lds(uint32_t max_child_ne, uint32_t max_nextv, uint32_t A);
 hipError_t launch_expand_small(const ExpandArgs& a, uint32_t grid_cap, uint32_t wpb, uint32_t lanes, hipStream_t st);
+// Large states of one arity 2..4 whose colours fit the LDS (hgx_wl_large.hpp): LDS per workgroup (all: with
+// every array, else the rest in large_scratch bytes of global memory per workgroup), and the
+// launches: W = 4, 8 or 16 waves per state, a.scratch set for the second layout.
+inline bool large_fits(uint32_t max_ne, uint32_t max_nextv, uint32_t A) {
+    return max_nextv <= kLargeMaxLabels && (uint64_t)max_ne * A * (A - 1) <= kLargeMaxEntries;
+}
+uint32_t large_lds(uint32_t max_ne, uint32_t max_nextv, uint32_t A, bool all);
+uint32_t large_scratch(uint32_t max_ne, uint32_t max_nextv, uint32_t A);
+hipError_t launch_expand_large(const ExpandArgs& a, uint32_t grid, uint32_t team, hipStream_t st);
+hipError_t launch_wl_large(const struct WLStatesArgs& a, uint32_t grid, uint32_t team, hipStream_t st);
 uint32_t expand_grid(uint32_t n_items, uint32_t team, uint32_t wpb, uint32_t grid_cap, uint32_t lanes = 64);
 // Records, identity and counters of the n children of a.M, whose hashes k_expand left in a.C.hash.
 hipError_t launch_record(const ExpandArgs& a, uint32_t n, hipStream_t st);

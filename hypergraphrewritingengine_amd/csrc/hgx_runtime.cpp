@@ -477,11 +477,41 @@ void sort_pairs_u64(Arena& ar, const uint64_t* kin, uint64_t* kout, const uint32
     HIP_TRY(hipcub::DeviceRadixSort::SortPairs(t, tmp, kin, kout, vin, vout, (int)n, 0, end_bit, st));
 }
 
+// Launch shape of the large-state hash: every array in LDS while that leaves a CU two workgroups, as many
+// workgroups as the CUs hold (four times as many where a workgroup keeps no global slice, so the last
+// ones even out), and the waves that share a state: few where there are states enough for the chip,
+// since waves past the work only add to the barriers, more for a long state or a few of them. Measured
+// with 4 / 8 / 16: k_expand of 20 k children of 256 to 2,048 edges 2.7 / 3.6 / 5.7 ms; of 360 children
+// of 2,500 edges 0.16 / 0.12 / 0.16, 4,000 0.29 / 0.20 / 0.25, 6,000 0.51 / 0.34 / 0.37, 9,000 1.36 /
+// 0.80 / 0.57, 12,001 2.15 / 1.25 / 0.89; one state of 2,500 edges 0.13 / 0.09 / 0.07, 12,001 0.87 /
+// 0.54 / 0.37. Everything in LDS at 6,000 edges (one workgroup a CU) 0.40 against 0.34 with 8.
+LargeShape large_shape(uint32_t max_ne, uint32_t max_nextv, uint32_t A, uint32_t n, uint32_t max_lds, uint32_t num_cu) {
+    LargeShape s;
+    s.all = large_lds(max_ne, max_nextv, A, true) <= max_lds / 2;
+    s.lds = large_lds(max_ne, max_nextv, A, s.all);
+    s.team = max_ne <= 2048 ? (n >= 4 * num_cu ? 4u : 8u) : max_ne > 7000 || n < num_cu / 8 ? 16u : 8u;
+    const uint32_t held = std::max(1u, std::min(max_lds / s.lds, 32u / s.team));
+    s.grid = launch_grid(n, 1, num_cu * held * (s.all ? 4u : 1u));
+    return s;
+}
+
 uint32_t place_wl_states(Arena& ar, WLStatesArgs& w, bool lean, uint32_t max_lds, uint32_t grid_cap,
                          uint32_t forced_team, uint32_t* wpb) {
     w.lean = lean && w.max_ne < 65536 ? 1u : 0u;
     w.lds_per_wave = wl_states_lds_per_wave(w.max_ne, w.max_nv, w.A, w.lean != 0);
     w.scratch = nullptr;
+    w.large = 0;
+    // past the one-wave workspaces, states whose colours fit the LDS (hgx_wl_large.hpp): one root of
+    // 12,001 edges 2.37 -> 0.37 ms
+    if (w.lean && w.A <= 4 && !forced_team && w.lds_per_wave > kTeamBytes[0] && large_fits(w.max_ne, w.max_nv, w.A) &&
+        large_lds(w.max_ne, w.max_nv, w.A, false) <= max_lds) {
+        const LargeShape sh = large_shape(w.max_ne, w.max_nv, w.A, w.n, max_lds, grid_cap / 8);
+        w.large = sh.grid;
+        w.lds_per_wave = sh.lds;
+        if (!sh.all) w.scratch = (uint8_t*)ar.alloc((size_t)sh.grid * large_scratch(w.max_ne, w.max_nv, w.A));
+        *wpb = 1;
+        return sh.team;
+    }
     const uint32_t team = pick_team(w.lds_per_wave, forced_team);
     if (team == 1) {
         *wpb = place_workspace(ar, w.lds_per_wave, w.n, max_lds, grid_cap, &w.scratch);

@@ -250,6 +250,11 @@ constexpr uint32_t kTeamBytes[2] = {24u << 10, 48u << 10};
 inline uint32_t pick_team(uint32_t bytes, uint32_t forced) {
     return forced ? forced : bytes <= kTeamBytes[0] ? 1u : bytes <= kTeamBytes[1] ? 4u : 8u;
 }
+struct LargeShape {
+    uint32_t lds, team, grid;    // LDS bytes per workgroup, waves per state, workgroups
+    bool all;                    // every array in LDS
+};
+LargeShape large_shape(uint32_t max_ne, uint32_t max_nextv, uint32_t A, uint32_t n, uint32_t max_lds, uint32_t num_cu);
 struct WLStatesArgs;
 // Workspace of a k_wl_states launch (lean when `lean`): sets lds_per_wave and scratch; returns
 // the team size, and the waves per workgroup in *wpb.

@@ -109,12 +109,12 @@ __device__ __forceinline__ uint32_t small_ndistinct(const TM& tm, const SmallSpa
                        const uint64_t hi_ = x[a] < x[b] ? x[b] : x[a]; x[a] = lo_; x[b] = hi_; }
 // Colour h folded with the values of a list of at most M entries in ascending order.
 template <int M>
-__device__ __forceinline__ uint64_t small_fold(const SmallSpace& s, const uint64_t* cur, uint32_t b, uint32_t n,
+__device__ __forceinline__ uint64_t small_fold(const uint16_t* nb, const uint64_t* cur, uint32_t b, uint32_t n,
                                                uint64_t h) {
     uint64_t x[M];
 #pragma unroll
     for (int i = 0; i < M; ++i) {
-        const uint32_t t = s.nb[(uint32_t)i < n ? b + i : b];
+        const uint32_t t = nb[(uint32_t)i < n ? b + i : b];
         const uint64_t val = fnv(cur[t >> 2], t & 3u);
         x[i] = (uint32_t)i < n ? val : ~0ull;
     }
@@ -298,11 +298,11 @@ __device__ __forceinline__ uint64_t wl_hash_small(const SmallSpace& s, const TM&
             uint64_t h = cur[v];
             // the smallest network that fits every lane here
             if (__ballot(n > 3) == 0)
-                h = __ballot(n > 2) == 0 ? small_fold<2>(s, cur, b, n, h) : small_fold<3>(s, cur, b, n, h);
+                h = __ballot(n > 2) == 0 ? small_fold<2>(s.nb, cur, b, n, h) : small_fold<3>(s.nb, cur, b, n, h);
             else if (__ballot(n > 6) == 0)
-                h = __ballot(n > 4) == 0 ? small_fold<4>(s, cur, b, n, h) : small_fold<6>(s, cur, b, n, h);
+                h = __ballot(n > 4) == 0 ? small_fold<4>(s.nb, cur, b, n, h) : small_fold<6>(s.nb, cur, b, n, h);
             else
-                h = small_fold<8>(s, cur, b, n, h);
+                h = small_fold<8>(s.nb, cur, b, n, h);
             nxt[v] = h;
         }
         tm.sync();
