@@ -502,17 +502,6 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
                     const int kc = (int)(&x - cls.data());
                     uint32_t team = pick_team(lpw(1), ctx_->join_team ? ctx_->join_team : ctx_->tune.join_team[kc]);
                     mc.lds_per_wave = lpw(team);
-                    uint32_t gws_grid = 0;
-                    if (lpw(8) > ctx_->max_lds) {
-                        // states whose workspace does not fit LDS: eight-wave teams over
-                        // per-workgroup slices of global memory (at most 2 per CU, 4 GiB in all)
-                        team = 8;
-                        mc.lds_per_wave = lpw(8);
-                        uint32_t cap = std::max<uint32_t>(8u, std::min<uint64_t>(2ull * ctx_->num_cu,
-                                                                                 (4ull << 30) / mc.lds_per_wave));
-                        gws_grid = launch_grid((uint32_t)x.n, 1, cap);
-                        mc.scratch = (uint8_t*)tmp.alloc((size_t)gws_grid * mc.lds_per_wave);
-                    }
                     if (x.n != n) {
                         uint32_t* d_r = dalloc<uint32_t>(tmp, x.rb.size() + x.rpre.size());
                         up(d_r, x.rb.data(), x.rb.size(), st);
@@ -534,6 +523,35 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
                         timed(ctx_, st, name, (uint64_t)((double)bytes * x.n / n), x.n,
                               [&] { return launch_match_bits(mc, emit, ctx_->num_cu * 32, wpb, st, lanes); }, kc);
                         continue;
+                    }
+                    // Larger binary states that fit the LDS: the join by lists per position, in full
+                    // unless forwarding is asked for (its merge costs more than this join). 8 waves
+                    // a state up to 2,048 edges, 16 above and where there are few (4 / 8 / 16:
+                    // served mix count 0.82 / 0.72 / 0.80 ms, emit 0.62 / 0.53 / 0.49; one state of
+                    // 2,500 edges 0.04 / 0.02 / 0.02, 12,001 0.16 / 0.08 / 0.06). Against k_match:
+                    // served mix 2.24 -> 0.72 and 1.55 -> 0.53, one state of 12,001 edges, in global
+                    // workspaces there, 1.43 -> 0.06 and 0.72 -> 0.11.
+                    const uint32_t lists = match_lists_lds(mc.max_ne, mc.max_nextv);
+                    if (x.uniform && ctx_->forward != 1 && !ctx_->join_team && lists <= ctx_->max_lds) {
+                        mc.fwd_n = 0; mc.dmax = 0;
+                        mc.lds_per_wave = lists;
+                        const uint32_t tw = mc.max_ne <= 2048 && x.n >= ctx_->num_cu ? 8u : 16u;
+                        const uint32_t held = std::max(1u, std::min(ctx_->max_lds / lists, 32u / tw));
+                        const uint32_t grid = launch_grid((uint32_t)x.n, 1, ctx_->num_cu * held * 4);
+                        timed(ctx_, st, name, (uint64_t)((double)bytes * x.n / n), x.n,
+                              [&] { return launch_match_lists(mc, emit, grid, tw, st); }, kc);
+                        continue;
+                    }
+                    uint32_t gws_grid = 0;
+                    if (lpw(8) > ctx_->max_lds) {
+                        // states whose workspace does not fit LDS: eight-wave teams over
+                        // per-workgroup slices of global memory (at most 2 per CU, 4 GiB in all)
+                        team = 8;
+                        mc.lds_per_wave = lpw(8);
+                        uint32_t cap = std::max<uint32_t>(8u, std::min<uint64_t>(2ull * ctx_->num_cu,
+                                                                                 (4ull << 30) / mc.lds_per_wave));
+                        gws_grid = launch_grid((uint32_t)x.n, 1, cap);
+                        mc.scratch = (uint8_t*)tmp.alloc((size_t)gws_grid * mc.lds_per_wave);
                     }
                     // sub-wave teams for small states, when the wave's workspaces fit a workgroup
                     uint32_t lanes = 64;

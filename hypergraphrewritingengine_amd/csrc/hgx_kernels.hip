@@ -3,6 +3,7 @@
 //   k_match<false>   SCAN -> EXPAND -> SINK join, counting matches per state
 //   k_match<true>    the same join, writing match records in the deterministic order
 //   k_match_bits     both over small binary states, by bit sets
+//   k_match_lists    both over larger binary states that fit the LDS, by lists per position
 //   k_expand         rewrite + WL hash, one team per child state
 //                    (k_expand_small: small children of one arity)
 //   k_record         each child's event, causal masks and records, its hash into its request's
@@ -925,6 +926,7 @@ __global__ __launch_bounds__(256) void k_match_bits(MatchArgs a) {
                 const bool ok = seed < ne && (!(J.bj[0] & 256u) || (sv & 0xFFu) == sv >> 8);
                 const uint32_t c = ok ? bit_join_any<NW, false>(J, n_lhs, seed, sv, RegJoinOut{}) : 0u;
                 mine += c;
+                if (capped && mine > budget) break;            // (count pass) the run is over its cap
                 if constexpr (EMIT) {
                     uint32_t round;
                     const uint32_t inc = tm.incl_scan(c, round);
@@ -979,6 +981,298 @@ hipError_t launch_match_bits(const MatchArgs& a, bool emit, uint32_t grid_cap, u
     return nw == 1 ? launch_match_bits_nw<1>(a, emit, grid, wpb, lanes, st)
            : nw == 2 ? launch_match_bits_nw<2>(a, emit, grid, wpb, lanes, st)
                      : launch_match_bits_nw<4>(a, emit, grid, wpb, lanes, st);
+}
+
+// ------------------------------------------------------------------------------------------
+// The join over larger binary states, up to what the LDS holds (8 bytes an edge and 4 a label), by the W
+// waves of a workgroup: the edges as vertex pairs in one word, and per (position, vertex) the list of
+// its edges. A depth takes the shorter list of its bound positions and tests the other one, its
+// binding words in registers (DRule::bj); a last depth with one bound position and nothing else to
+// test counts its list's length less the edges in use. Matches and their order are k_match's: the
+// emit pass puts every list in edge order. What bounded k_match here were the chains of LDS reads per
+// candidate, and for states past its 25 bytes an edge of LDS a workspace in global memory.
+// ------------------------------------------------------------------------------------------
+
+struct ListJoin {
+    const uint32_t* ev;        // edges: first vertex | second << 16
+    const uint32_t* end;       // per vertex: end of its list at position 0 | at position 1 << 16
+    const uint16_t* l0;
+    const uint16_t* l1;
+    uint32_t ne;
+    uint32_t bj[4];
+};
+
+template <int N, int D, bool OUT>
+__device__ __forceinline__ uint32_t list_join(const ListJoin& J, Bound B, const RegJoinOut& o, uint32_t found) {
+    if constexpr (D == N) {
+        if constexpr (OUT) {
+            const size_t at = (size_t)(o.base + found);
+            uint16_t* q = o.q + at * o.K;
+            q[(J.bj[0] >> 12) & 3u] = (uint16_t)B.e0;
+            if (N > 1) q[(J.bj[1] >> 12) & 3u] = (uint16_t)B.e1;
+            if (N > 2) q[(J.bj[2] >> 12) & 3u] = (uint16_t)B.e2;
+            if (N > 3) q[(J.bj[3] >> 12) & 3u] = (uint16_t)B.e3;
+            o.parent[at] = o.state; o.rule[at] = o.rule_id; o.cne[at] = o.child_ne;
+        }
+        return found + 1;
+    } else {
+        const uint32_t b = J.bj[D];
+        auto value = [&](uint32_t src) {                 // a bound position's vertex
+            const uint32_t d = (src >> 1) & 3u;
+            uint32_t x = B.v0;
+            if (D > 1) { const uint32_t m = 0u - (uint32_t)(d == 1); x = (x & ~m) | (B.v1 & m); }
+            if (D > 2) { const uint32_t m = 0u - (uint32_t)(d == 2); x = (x & ~m) | (B.v2 & m); }
+            return (src & 8u) ? x >> 16 : x & 0xFFFFu;
+        };
+        const bool b0 = (b & 1u) != 0, b1 = (b & 16u) != 0, rep = (b & 256u) != 0;
+        const uint32_t x0 = b0 ? value(b) : 0u, x1 = b1 ? value(b >> 4) : 0u;
+        uint32_t lo = 0, hi = J.ne;
+        const uint16_t* list = nullptr;
+        if (b0) {
+            lo = x0 ? J.end[x0 - 1] & 0xFFFFu : 0u;
+            hi = J.end[x0] & 0xFFFFu;
+            list = J.l0;
+        }
+        if (b1) {
+            const uint32_t lo1 = x1 ? J.end[x1 - 1] >> 16 : 0u, hi1 = J.end[x1] >> 16;
+            if (!b0 || hi1 - lo1 < hi - lo) { lo = lo1; hi = hi1; list = J.l1; }
+        }
+        if constexpr (D + 1 == N && !OUT) {
+            if (b0 != b1 && !rep) {
+                // the list less the edges in use that are on it
+                auto on = [&](uint32_t v) { return b0 ? (v & 0xFFFFu) == x0 : v >> 16 == x1; };
+                uint32_t c = hi - lo - (on(B.v0) ? 1u : 0u);
+                if (D > 1) c -= on(B.v1) ? 1u : 0u;
+                if (D > 2) c -= on(B.v2) ? 1u : 0u;
+                return found + c;
+            }
+        }
+        for (uint32_t j = lo; j < hi; ++j) {
+            const uint32_t e = list ? (uint32_t)list[j] : j;
+            const uint32_t v = J.ev[e];
+            bool ok = e != B.e0;
+            if (D > 1) ok &= e != B.e1;
+            if (D > 2) ok &= e != B.e2;
+            ok &= !b0 || (v & 0xFFFFu) == x0;
+            ok &= !b1 || v >> 16 == x1;
+            ok &= !rep || (v & 0xFFFFu) == v >> 16;
+            if (!ok) continue;
+            B.template set<D>(e, v);
+            found = list_join<N, D + 1, OUT>(J, B, o, found);
+        }
+        return found;
+    }
+}
+
+template <bool OUT>
+__device__ __forceinline__ uint32_t list_join_any(const ListJoin& J, uint32_t n_lhs, uint32_t seed, uint32_t sv,
+                                                  const RegJoinOut& o) {
+    const Bound B{seed, 0, 0, 0, sv, 0, 0, 0};
+    switch (n_lhs) {
+        case 1: return list_join<1, 1, OUT>(J, B, o, 0u);
+        case 2: return list_join<2, 1, OUT>(J, B, o, 0u);
+        case 3: return list_join<3, 1, OUT>(J, B, o, 0u);
+        default: return list_join<4, 1, OUT>(J, B, o, 0u);
+    }
+}
+
+// Workspace: edges, list ends, the two lists, a bit per edge and the lists above 16 entries (emit).
+struct ListSizes {
+    uint32_t NE, NL, NB, NH;
+    __host__ __device__ static ListSizes make(uint32_t ne, uint32_t nl) {
+        return ListSizes{ne, nl, (ne + 31) / 32, 2 * ne / 17 + 1};
+    }
+    __host__ __device__ uint32_t bytes() const {
+        auto al = [](uint32_t b) { return (b + 7u) & ~7u; };
+        return al(4 * NE) + al(4 * (NL + 1)) + 2 * al(2 * NE) + al(4 * NB) + al(4 * NH) + 16 + 128;
+    }
+};
+
+// The list [lo, hi) of l into ascending order (edge ids are distinct), by the workgroup: marked in a bit
+// set and read back in order.
+template <class TM>
+__device__ __forceinline__ void sort_list_bits(const TM& tm, uint16_t* l, uint32_t lo, uint32_t hi, uint32_t* bits,
+                                               uint32_t nb) {
+    for (uint32_t i = tm.r; i < nb; i += TM::N) bits[i] = 0;
+    tm.sync();
+    for (uint32_t j = lo + tm.r; j < hi; j += TM::N) atomicOr(&bits[l[j] >> 5], 1u << (l[j] & 31u));
+    tm.sync();
+    uint32_t at = lo;
+    for (uint32_t base = 0; base < nb; base += TM::N) {
+        const uint32_t i = base + tm.r;
+        uint32_t w = i < nb ? bits[i] : 0u, round;
+        uint32_t o = (uint32_t)__popc(w);
+        o = at + tm.incl_scan(o, round) - o;
+        for (; w; w &= w - 1) l[o++] = (uint16_t)(i * 32 + (uint32_t)__builtin_ctz(w));
+        at += round;
+    }
+    tm.sync();
+}
+
+template <bool EMIT, uint32_t W>
+__global__ __launch_bounds__(64 * W) void k_match_lists(MatchArgs a) {
+    extern __shared__ uint8_t lds[];
+    constexpr uint32_t N = 64 * W;
+    const ListSizes z = ListSizes::make(a.max_ne, a.max_nextv);
+    uint8_t* p = lds;
+    uint32_t* ev = (uint32_t*)carve(p, 4 * z.NE);
+    uint32_t* end = (uint32_t*)carve(p, 4 * (z.NL + 1));
+    uint16_t* l0 = (uint16_t*)carve(p, 2 * z.NE);
+    uint16_t* l1 = (uint16_t*)carve(p, 2 * z.NE);
+    uint32_t* bits = (uint32_t*)carve(p, 4 * z.NB);
+    uint32_t* hubs = (uint32_t*)carve(p, 4 * z.NH);
+    uint32_t* word = (uint32_t*)carve(p, 16);
+    const Team<W> tm((uint64_t*)carve(p, 128));
+    const uint32_t l = tm.r, A = a.P.A;
+    const uint32_t n_items = a.nrange ? a.n_items : a.P.n;
+    const bool spread = !EMIT && a.spread > 1;
+    const uint32_t nblk = (n_items + kCountSpreadBlock - 1) / kCountSpreadBlock;
+    const uint32_t n_loop = spread ? nblk * kCountSpreadBlock : n_items;
+    for (uint32_t ls = blockIdx.x; ls < n_loop; ls += gridDim.x) {
+        uint32_t s = ls;
+        if (spread) {
+            s = (uint32_t)((uint64_t)(ls / kCountSpreadBlock) * a.spread % nblk) * kCountSpreadBlock +
+                ls % kCountSpreadBlock;
+            if (s >= n_items) continue;                         // the last block's tail
+        }
+        if (a.nrange) {                                         // subset: logical -> state
+            uint32_t lo = 0, hi = a.nrange;
+            while (hi - lo > 1) { const uint32_t mid = (lo + hi) >> 1; if (a.rpre[mid] <= s) lo = mid; else hi = mid; }
+            s = a.rb[lo] + (s - a.rpre[lo]);
+        }
+        const uint32_t run = a.P.run[s];
+        const uint32_t ne = a.P.ne[s];
+        const uint64_t eo = a.P.eoff[s];
+        const uint32_t nvid = a.P.nextv[s];                     // labels are < nvid
+        const uint8_t active = a.active[run] && (!a.smask || a.smask[s]);
+        const uint64_t budget = EMIT ? 0 : (uint64_t)a.budget[run];
+        const bool capped = !EMIT && budget != kNoBudget;
+        // one read of the run's tally, which moves under other workgroups, for all of the team
+        const uint64_t tally = capped ? tm.bcast(l == 0 ? (uint64_t)a.run_acc[run] : 0ull) : 0ull;
+        if (!active || (EMIT ? a.cnt[s] == 0 : tally > budget)) {
+            if (!EMIT && l == 0) { a.cnt[s] = 0; a.state_edges[s] = 0; }
+            continue;
+        }
+        tm.sync();
+        for (uint32_t v = l; v <= nvid; v += N) end[v] = 0;
+        if (l == 0) word[0] = 0;
+        tm.sync();
+        for (uint32_t e = l; e < ne; e += N) {
+            uint32_t x, y;
+            if (A == 2) { const uint2 v = ((const uint2*)a.P.ev)[eo + e]; x = v.x; y = v.y; }
+            else { x = a.P.ev[(eo + e) * A]; y = a.P.ev[(eo + e) * A + 1]; }
+            ev[e] = x | y << 16;
+            atomicAdd(&end[x], 1u);
+            atomicAdd(&end[y], 1u << 16);
+        }
+        tm.sync();
+        tm.excl_scan_lds(end, nvid + 1);        // both positions' counts at once: neither sum passes 16 bits
+        for (uint32_t e = l; e < ne; e += N) {
+            const uint32_t v = ev[e];
+            l0[atomicAdd(&end[v & 0xFFFFu], 1u) & 0xFFFFu] = (uint16_t)e;
+            l1[atomicAdd(&end[v >> 16], 1u << 16) >> 16] = (uint16_t)e;
+        }
+        tm.sync();
+        if constexpr (EMIT) {
+            // every list into edge order: up to 16 entries by a lane, to 64 by a wave, longer ones by
+            // the workgroup
+            for (uint32_t i = l; i < 2 * nvid; i += N) {
+                const uint32_t v = i >> 1, sh = (i & 1u) * 16;
+                const uint32_t lo = v ? (end[v - 1] >> sh) & 0xFFFFu : 0u, hi = (end[v] >> sh) & 0xFFFFu;
+                if (hi - lo < 2) continue;
+                if (hi - lo > 16) { hubs[atomicAdd(&word[0], 1u)] = i; continue; }
+                uint16_t* q = sh ? l1 : l0;
+                for (uint32_t j = lo + 1; j < hi; ++j) {
+                    const uint16_t x = q[j];
+                    uint32_t k = j;
+                    while (k > lo && q[k - 1] > x) { q[k] = q[k - 1]; --k; }
+                    q[k] = x;
+                }
+            }
+            tm.sync();
+            const uint32_t nh = word[0];
+            for (uint32_t k = l / WAVE; k < nh; k += W) {
+                const uint32_t i = hubs[k], v = i >> 1, sh = (i & 1u) * 16;
+                const uint32_t lo = v ? (end[v - 1] >> sh) & 0xFFFFu : 0u, n = ((end[v] >> sh) & 0xFFFFu) - lo;
+                if (n > WAVE) continue;
+                uint16_t* q = sh ? l1 : l0;
+                const uint32_t ln = lane_id(), un = (uint32_t)__builtin_amdgcn_readfirstlane((int)n);
+                const uint32_t x = ln < n ? q[lo + ln] : 0xFFFFFFFFu;
+                uint32_t r = 0;
+                for (uint32_t j = 0; j < un; ++j) r += (uint32_t)__builtin_amdgcn_readlane((int)x, (int)j) < x ? 1u : 0u;
+                if (ln < n) q[lo + r] = (uint16_t)x;
+            }
+            for (uint32_t k = 0; k < nh; ++k) {
+                const uint32_t i = hubs[k], v = i >> 1, sh = (i & 1u) * 16;
+                const uint32_t lo = v ? (end[v - 1] >> sh) & 0xFFFFu : 0u, hi = (end[v] >> sh) & 0xFFFFu;
+                if (hi - lo > WAVE) sort_list_bits(tm, sh ? l1 : l0, lo, hi, bits, (ne + 31) / 32);
+            }
+            tm.sync();
+        }
+        const DRun& RN = a.runs[run];
+        ListJoin J;
+        J.ev = ev; J.end = end; J.l0 = l0; J.l1 = l1; J.ne = ne;
+        uint32_t total = 0;
+        uint64_t edges_sum = 0;                                // count pass: edges of the children
+        uint32_t out = EMIT ? (uint32_t)a.moff[s] : 0u;
+        for (uint32_t r = 0; r < RN.n_rules; ++r) {
+            const DRule& R = RN.rules[r];
+            if (!R.bits_ok) continue;                           // a pattern edge that is not binary
+            const uint32_t n_lhs = R.n_lhs, child_ne = ne - n_lhs + R.n_rhs;
+#pragma unroll
+            for (int d = 0; d < 4; ++d) J.bj[d] = R.bj[d];
+            uint32_t mine = 0;
+            for (uint32_t base = 0; base < ne; base += N) {
+                const uint32_t seed = base + l;
+                const uint32_t sv = seed < ne ? ev[seed] : 0u;
+                const bool ok = seed < ne && (!(J.bj[0] & 256u) || (sv & 0xFFFFu) == sv >> 16);
+                const uint32_t c = ok ? list_join_any<false>(J, n_lhs, seed, sv, RegJoinOut{}) : 0u;
+                mine += c;
+                if (capped && mine > budget) break;            // (count pass) the run is over its cap
+                if constexpr (EMIT) {
+                    uint32_t round;
+                    const uint32_t inc = tm.incl_scan(c, round);
+                    if (c) {
+                        const RegJoinOut ro{a.M.q, a.M.K, out + inc - c, a.M.parent, a.M.rule, a.M.cne, s, r, child_ne};
+                        list_join_any<true>(J, n_lhs, seed, sv, ro);
+                    }
+                    out += round;
+                }
+            }
+            if constexpr (!EMIT) {
+                const uint32_t sum = tm.sum(mine);
+                total += sum;
+                edges_sum += (uint64_t)sum * child_ne;
+            }
+        }
+        if (!EMIT && l == 0) {
+            a.cnt[s] = total;
+            a.state_edges[s] = edges_sum;
+            if (total && capped) atomicAdd(&a.run_acc[run], (unsigned long long)total);
+        }
+    }
+}
+
+uint32_t match_lists_lds(uint32_t max_ne, uint32_t max_nextv) {
+    return (ListSizes::make(max_ne, max_nextv).bytes() + 15u) & ~15u;
+}
+
+hipError_t launch_match_lists(const MatchArgs& a, bool emit, uint32_t grid, uint32_t team, hipStream_t st) {
+    const uint32_t items = a.nrange ? a.n_items : a.P.n;
+    if (!items) return hipSuccess;
+    if (a.max_ne > 65535 || a.max_nextv > 65535 || a.scratch || a.fwd_n || a.P.A < 2) return hipErrorInvalidValue;
+    const dim3 g(grid);
+    const size_t lds = a.lds_per_wave;
+    switch (team * 2 + (emit ? 1 : 0)) {
+        case 8: hipLaunchKernelGGL((k_match_lists<false, 4>), g, dim3(256), lds, st, a); break;
+        case 9: hipLaunchKernelGGL((k_match_lists<true, 4>), g, dim3(256), lds, st, a); break;
+        case 16: hipLaunchKernelGGL((k_match_lists<false, 8>), g, dim3(512), lds, st, a); break;
+        case 17: hipLaunchKernelGGL((k_match_lists<true, 8>), g, dim3(512), lds, st, a); break;
+        case 32: hipLaunchKernelGGL((k_match_lists<false, 16>), g, dim3(1024), lds, st, a); break;
+        case 33: hipLaunchKernelGGL((k_match_lists<true, 16>), g, dim3(1024), lds, st, a); break;
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
 }
 
 // ------------------------------------------------------------------------------------------
