@@ -12,25 +12,59 @@
 
 namespace hgx {
 
+// Lists of at most kIndexShort entries are ordered by a thread per entry that counts, of at most
+// kIndexWave by a wave per list that counts in LDS (cost n^2 / 64), longer ones by a bit set of the
+// edges in LDS (cost of all edges / 32, whatever n). States of at most kIndexPlaceEdges edges have their lists placed and ordered rather
+// than sorted: the bit set of 2^20 edges is 128 KB, and the two ways meet there -- wedges of random
+// graphs (edges / 10 vertices), whole join: 98 against 128 us at 20,000 edges, 237 / 339 at 500,000,
+// 350 / 462 at 1 million, 589 / 600 at 2 million and 1,017 / 966 at 4 million (placed / sorted).
+constexpr uint32_t kIndexShort = 32;
+constexpr uint32_t kIndexWave = 256;
+constexpr uint32_t kIndexPlaceEdges = 1u << 20;
+
 struct BJView {
     DRule R;
     const uint32_t* ev;     // [m * A]
     const uint8_t* ar;      // [m]
     uint32_t m, A;
-    const uint32_t* off;    // [nkeys + 1]
-    const uint32_t* idx;    // [occurrences]
-    // Closing edges: a depth whose pattern edge has every vertex bound by earlier depths takes
-    // its candidates from the edges with exactly that vertex tuple -- the edges sorted by a
-    // 64-bit key of (arity, vertices), stably, so equal keys stay in edge order. Bit d of
-    // `full` marks such a depth (0: no tuple index).
-    const uint64_t* tkey;   // [m] sorted keys
-    const uint32_t* tidx;   // [m] edges in key order
-    uint32_t full;
-    // Each distinct key's run [lo, lo + cnt) of tidx, in an open-addressing table (key 0 empty;
-    // a zero key is stored as 1, which only widens its run's verification)
-    uint64_t* tslot;        // [tmask + 1] keys
-    uint2* trun;            // [tmask + 1] (lo, cnt)
-    uint32_t tmask;
+    // The CSR over the U positions the join pivots on: list vertex * U + u holds, ascending, the
+    // edges with the vertex at position upos[u] and an arity in the bit set uar[u].
+    uint32_t U;
+    uint8_t upos[16];
+    uint8_t dpos[16];       // per depth: which of them it pivots on
+    uint32_t uar[16];
+    const uint32_t* off;    // [lists + 1]
+    const uint32_t* idx;    // [entries]
+    // What a depth compares of a candidate: the slots, and (bit d of chk_ar) the arity
+    uint32_t chk[16];
+    uint32_t chk_ar;
+    // Closing edges: a depth whose pattern edge has every vertex bound by earlier depths takes its
+    // candidates from the edges with exactly that vertex tuple, by an open-addressing table of
+    // 32-bit tags (0 empty; a tag shared by two tuples only widens a list's verification). The
+    // edges of the tuple at place h are tidx[toff[h] - toff[0] ..], ascending. Bit d of `full`
+    // marks such a depth (0: no table), tar is the bit set of their arities.
+    uint32_t full, tar, tmask;
+    const uint32_t* tslot;  // [tmask + 1]
+    const uint32_t* toff;   // [tmask + 2]
+    const uint32_t* tidx;
+};
+
+// The index while it is built.
+struct BJIndex {
+    uint32_t nkeys;         // lists of the CSR
+    uint64_t tcnt0, scnt0;  // where the tuples' and the seeds' counts begin in cnt
+    uint32_t* cnt;          // counts: lists + 1, (tuple table + 1,) workgroups' seeds + 1
+    uint32_t* rank;         // [m * U] an entry's place in its list; its list (sorted instead)
+    uint32_t* tplace;       // [m] a tuple's place in the table
+    uint32_t* trank;        // [m] the edge's place in the tuple's list
+    uint32_t* tslot;
+    uint32_t* un;           // [m * U + m] list entries in arrival order, tuples' from tbase
+    uint32_t* idx;          //   and ascending
+    uint32_t tbase;
+    uint32_t* longq;        // lists of more than kIndexWave entries (tuple h: nkeys + 1 + h)
+    uint64_t* smask;        // one bit per edge: a seed
+    uint32_t* seeds;
+    uint32_t* scal;         // seeds, longest list, long lists, longest tuple list
 };
 
 // Device memory of one join: an Arena, or a fixed region (the allocation-free entry point)
@@ -50,6 +84,8 @@ struct BJMem {
     }
     size_t mark() const { return used; }
     void rewind(size_t m) { if (!arena) used = m; }
+    // bytes a depth's tiles may take before it splits its partials in two
+    size_t left() const { return arena ? ((size_t)1 << 30) : (cap > used + (1u << 20) ? cap - used - (1u << 20) : 0); }
     // bytes a next frontier may take before the depth splits its partials in two
     size_t room() const { return arena ? ((size_t)1 << 30) : (cap > used + (8u << 20) ? cap - used - (8u << 20) : 0); }
 };
@@ -63,7 +99,8 @@ struct BJRun {
     uint64_t cap = 0;
     uint64_t found = 0;
     uint32_t maxlist = 0;     // the longest candidate list of the index
-    uint64_t* acc = nullptr;  // device: matches found, join bytes (written by the depths)
+    uint64_t* acc = nullptr;  // device: matches found (by turns, two), join bytes
+    uint32_t turn = 0;        // which of the two holds the matches found so far
     uint64_t index_bytes = 0; // algorithmic bytes of the index build
     uint64_t alg_bytes = 0;   // of the join: adjacency reads of every item, frontiers, matches
 };
