@@ -8,7 +8,8 @@
 // (the counter's old value is an entry's place in its list), marks the seeds, and counts the edges
 // of each vertex tuple in a hash table (for closing edges, below); one scan places lists, tuples
 // and seeds; a second pass writes the entries, and a third puts each list in ascending order by
-// counting an entry's smaller neighbours (long lists in LDS, the longest by a bit set of the edges there). Above
+// counting an entry's smaller neighbours (long lists in LDS, the longest by a bit set of the edges
+// there). Above
 // kIndexPlaceEdges edges the lists come from a stable radix sort of (list, edge) pairs instead.
 //
 // Join (join_core.hpp:143-208), breadth first: the partial matches of depth d (d edges in join

@@ -24,7 +24,8 @@ static double ms_since(Clock::time_point t) {
     return std::chrono::duration<double, std::milli>(Clock::now() - t).count();
 }
 
-Engine::Engine(hgx_ctx* ctx) : ctx_(ctx), st_(ctx->stream), pool_(ctx->pool), slab_(ctx->pool.get()) {
+Engine::Engine(hgx_ctx* ctx)
+    : ctx_(ctx), st_(ctx->stream), pool_(ctx->pool), slab_(ctx->pool.get()), stage_owner_(ctx->stage) {
     grow_slots(256);
 }
 
@@ -40,17 +41,81 @@ void Engine::set_mode(EngineMode m, std::shared_ptr<PassPlan> plan, uint32_t* ch
     d_check_ = check;
 }
 
+// Staging holds a transfer's bytes and, at its flush, one Move per kMoveBytes of them.
+uint8_t* Engine::stage(size_t bytes) {
+    const size_t need = ((bytes + 15) & ~(size_t)15);
+    const size_t moves = sizeof(Move) * (moves_.size() + bytes / kMoveBytes + 2);
+    if (stage_used_ + need + moves > stage_size_) {
+        if (mode_ == EngineMode::Capture) {
+            if (!moves_.empty()) return nullptr;              // (their Moves need the room)
+            stage_size_ = std::max<size_t>((size_t)1 << 20, 2 * need + moves);
+            void* h = nullptr;
+            HIP_TRY(hipHostMalloc(&h, stage_size_, hipHostMallocDefault));
+            pinned_.push_back(h);
+            stage_p_ = (uint8_t*)h;
+            stage_used_ = 0;
+        } else {
+            if (lease_) return nullptr;
+            lease_ = std::make_unique<StageLease>(*stage_owner_);
+            stage_p_ = lease_->half(0);
+            stage_size_ = 2 * StageLease::kHalf;
+            if (need + moves > stage_size_) return nullptr;
+        }
+    }
+    uint8_t* p = stage_p_ + stage_used_;
+    stage_used_ += need;
+    return p;
+}
+
 void Engine::put(void* dst, const void* src, size_t bytes, hipStream_t st) {
     if (!bytes) return;
-    if (mode_ != EngineMode::Capture) {
-        HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st));
-        return;
+    const bool capture = mode_ == EngineMode::Capture;
+    if (bytes <= kMoveMax || capture) {
+        uint8_t* p = stage(bytes);
+        if (!p && capture) { flush(st); p = stage(bytes); }
+        if (p) {
+            std::memcpy(p, src, bytes);
+            for (size_t o = 0; o < bytes; o += kMoveBytes)
+                moves_.push_back(Move{(uint8_t*)dst + o, p + o, std::min<uint64_t>(kMoveBytes, bytes - o)});
+            return;
+        }
     }
-    void* h = nullptr;
-    HIP_TRY(hipHostMalloc(&h, bytes, hipHostMallocDefault));
-    pinned_.push_back(h);
-    std::memcpy(h, src, bytes);
-    HIP_TRY(hipMemcpyAsync(dst, h, bytes, hipMemcpyHostToDevice, st));
+    HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st));
+}
+
+void Engine::get(void* dst, const void* src, size_t bytes, hipStream_t st) {
+    if (!bytes) return;
+    if (bytes <= kMoveMax)
+        if (uint8_t* p = stage(bytes)) {
+            for (size_t o = 0; o < bytes; o += kMoveBytes)
+                moves_.push_back(Move{p + o, (const uint8_t*)src + o, std::min<uint64_t>(kMoveBytes, bytes - o)});
+            fetches_.push_back(Fetch{dst, p, bytes});
+            return;
+        }
+    HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st));
+}
+
+void Engine::flush(hipStream_t st) {
+    if (moves_.empty()) return;
+    Move* m = (Move*)(stage_p_ + stage_used_);
+    std::memcpy(m, moves_.data(), sizeof(Move) * moves_.size());
+    stage_used_ += (sizeof(Move) * moves_.size() + 15) & ~(size_t)15;
+    HIP_TRY(launch_move(m, (uint32_t)moves_.size(), st));
+    moves_.clear();
+}
+
+void Engine::settle(hipStream_t st) {
+    flush(st);
+    HIP_TRY(hipStreamSynchronize(st));
+    for (const Fetch& f : fetches_) std::memcpy(f.dst, f.from, f.bytes);
+    fetches_.clear();
+    if (mode_ != EngineMode::Capture) stage_used_ = 0;
+}
+
+void Engine::drop_moves() {
+    moves_.clear();
+    fetches_.clear();
+    if (mode_ != EngineMode::Capture) stage_used_ = 0;
 }
 
 void Engine::fill_counts(RunRec& r, const uint64_t* x) {
@@ -200,8 +265,8 @@ void Engine::finalize(std::vector<std::shared_ptr<RunRec>>& runs) {
         return;
     }
     std::vector<uint64_t> ctr((size_t)hw_slots_ * CTR_N);       // slots ever taken
-    d2h(ctr.data(), d_ctr_, ctr.size(), st_);
-    HIP_TRY(hipStreamSynchronize(st_));
+    down(ctr.data(), d_ctr_, ctr.size(), st_);
+    settle(st_);
     for (auto& r : runs) {
         fill_counts(*r, &ctr[(size_t)r->slot * CTR_N]);
         r->t_done = now;
@@ -223,6 +288,7 @@ struct ExpandClass {
     bool uniform = true;                      // every request of the class has one arity 2..4
     uint64_t n = 0;
     std::vector<uint32_t> rb, rpre{0};
+    uint32_t* d_rb = nullptr;                 // on the device, rpre after rb (a class of part of the items)
 };
 constexpr uint32_t kClassEdges[6] = {32, 64, 128, 512, 2048, 0xFFFFFFFFu};
 // The expansion's size classes are finer at the small end, where a child's workspace is a few KiB
@@ -276,6 +342,10 @@ uint32_t coprime_stride(uint32_t n) {
 }  // namespace
 
 uint32_t Engine::step() {
+    if (!moves_.empty() || !fetches_.empty()) {     // left by a step that failed
+        HIP_TRY(hipStreamSynchronize(st_));
+        drop_moves();
+    }
     // runs of the frontier still evolving, and the counters before this generation touches them
     bool frontier_live = false;
     for (auto& r : F_runs_) frontier_live |= !r->done && live_.count(r->id) != 0;
@@ -307,6 +377,7 @@ uint32_t Engine::step() {
 void Engine::recover(const std::string& why, std::vector<std::shared_ptr<RunRec>>& admitted, bool frontier_live) {
     (void)hipStreamSynchronize(st_);
     (void)hipGetLastError();
+    drop_moves();
     if (frontier_live && hw_slots_)
         HIP_TRY(hipMemcpyAsync(d_ctr_, d_ctr_snap_, sizeof(uint64_t) * hw_slots_ * CTR_N,
                                hipMemcpyDeviceToDevice, st_));
@@ -373,7 +444,6 @@ void Engine::recover(const std::string& why, std::vector<std::shared_ptr<RunRec>
     release_next_.clear();
 }
 
-void frontier_ir(const DevGen& G, uint32_t b, uint32_t e, hipStream_t st, RunRec& r);
 
 uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
     const auto t_step = Clock::now();
@@ -388,6 +458,17 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
     std::vector<uint64_t> tot(nF, 0);
     uint64_t M = 0, parent_edges = 0;
     uint32_t K = 1;
+    // the ranges of all of a pass's classes (none for one class of all `items`), with whatever
+    // else is staged for the pass
+    auto put_ranges = [&](auto& cls, uint64_t items) {
+        for (auto& x : cls) {
+            if (!x.n || x.n == items) continue;
+            x.d_rb = dalloc<uint32_t>(tmp, x.rb.size() + x.rpre.size());
+            up(x.d_rb, x.rb.data(), x.rb.size(), st);
+            up(x.d_rb + x.rb.size(), x.rpre.data(), x.rpre.size(), st);
+        }
+        flush(st);
+    };
     MatchView mv{};
     uint32_t* cnt = nullptr;
     uint64_t* moff = nullptr;
@@ -488,6 +569,7 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
                     x.n += F_e_[i] - F_b_[i];
                     x.rpre.push_back((uint32_t)x.n);
                 }
+                put_ranges(cls, n);
                 for (auto& x : cls) {
                     if (!x.n) continue;
                     MatchArgs mc = ma;
@@ -503,10 +585,7 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
                     uint32_t team = pick_team(lpw(1), ctx_->join_team ? ctx_->join_team : ctx_->tune.join_team[kc]);
                     mc.lds_per_wave = lpw(team);
                     if (x.n != n) {
-                        uint32_t* d_r = dalloc<uint32_t>(tmp, x.rb.size() + x.rpre.size());
-                        up(d_r, x.rb.data(), x.rb.size(), st);
-                        up(d_r + x.rb.size(), x.rpre.data(), x.rpre.size(), st);
-                        mc.rb = d_r; mc.rpre = d_r + x.rb.size(); mc.nrange = (uint32_t)x.rb.size();
+                        mc.rb = x.d_rb; mc.rpre = x.d_rb + x.rb.size(); mc.nrange = (uint32_t)x.rb.size();
                         mc.n_items = (uint32_t)x.n;
                     }
                     if (!emit)
@@ -583,10 +662,11 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
                 rb = plan_->rb[plan_rb_++];
                 uint64_t* want = dalloc<uint64_t>(tmp, cap_slots_);
                 up(want, rb.data() + cap_slots_, cap_slots_, st);
+                flush(st);
                 HIP_TRY(launch_plan_check(d_tot_, want, d_budget_, cap_slots_, d_check_, st));
             } else {
-                d2h(rb.data(), d_run_edges_, rb.size(), st);
-                HIP_TRY(hipStreamSynchronize(st));
+                down(rb.data(), d_run_edges_, rb.size(), st);
+                settle(st);
                 if (mode_ == EngineMode::Record) plan_->rb.push_back(rb);
             }
             t_count = ms_since(t_step);
@@ -671,6 +751,7 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
             }
             if (masked) {
                 up(d_active_, h_active.data(), cap_slots_, st);
+                flush(st);
                 HIP_TRY(launch_mask_counts(F_->v.run, d_active_, n, cnt, st));
                 scan_u32_to_u64(tmp, cnt, moff, n, st);
             }
@@ -752,6 +833,7 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
         AdmitItem* d_items = dalloc<AdmitItem>(tmp, a_items.size());
         if (nh) up(d_stage, a_rules.data(), a_rules.size(), st);
         up(d_items, a_items.data(), a_items.size(), st);
+        flush(st);
         HIP_TRY(launch_admit(d_items, (uint32_t)a_items.size(), d_ctr_, st));
     }
 
@@ -874,6 +956,7 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
                 x.n += ce[i] - cb[i];
                 x.rpre.push_back((uint32_t)x.n);
             }
+            put_ranges(cls, M);
             const uint64_t bytes = M * (8ull + 2ull * K) + parent_edges * (4ull * F_->v.A + 2) +
                                    EC * (4ull * A + 2) + M * 8ull;
             for (int k = 0; k < kExpandClasses; ++k) {
@@ -888,10 +971,7 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
                 ea.lds_per_wave = expand_lds_per_wave(ea.max_child_ne, ea.max_nv, ea.max_nextv, A, ea.lean != 0);
                 ea.n_items = (uint32_t)x.n;
                 if (x.n != M) {
-                    uint32_t* d_r = dalloc<uint32_t>(tmp, x.rb.size() + x.rpre.size());
-                    up(d_r, x.rb.data(), x.rb.size(), st);
-                    up(d_r + x.rb.size(), x.rpre.data(), x.rpre.size(), st);
-                    ea.rb = d_r; ea.rpre = d_r + x.rb.size(); ea.nrange = (uint32_t)x.rb.size();
+                    ea.rb = x.d_rb; ea.rpre = x.d_rb + x.rb.size(); ea.nrange = (uint32_t)x.rb.size();
                 }
                 if (ea.lean && ea.max_child_ne <= kSmallMaxEdges && ea.max_nextv <= kSmallMaxLabels &&
                     ctx_->expand_team <= 1) {
@@ -993,8 +1073,10 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
                 }
                 RootCopy* d_copy = dalloc<RootCopy>(tmp, r_copy.size());
                 up(d_copy, r_copy.data(), r_copy.size(), st);
+                flush(st);
                 HIP_TRY(launch_copy_roots(d_copy, (uint32_t)r_copy.size(), v, st));
             }
+            flush(st);
             uint32_t rmax_ne = 1, rmax_nv = 1;
             for (auto& r : admitted) {
                 rmax_ne = std::max(rmax_ne, r->hp->max_root_ne);
@@ -1033,6 +1115,7 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
                     HIP_TRY(hipMemcpyAsync(bcnt, cnt, sizeof(uint32_t) * (n + 1), hipMemcpyDeviceToDevice, st));
                     uint8_t* d_bf = dalloc<uint8_t>(tmp, cap_slots_);
                     up(d_bf, bflag.data(), cap_slots_, st);
+                    flush(st);
                     HIP_TRY(launch_mask_counts(F_->v.run, d_bf, n, bcnt, st));
                     if (mode_ != EngineMode::Capture) HIP_TRY(hipStreamSynchronize(st));
                 }
@@ -1088,8 +1171,8 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
                             throw Error{HGX_ERR_INVALID, "the pass being captured left its recording"};
                         h_poff = plan_->poff[plan_poff_++];
                     } else {
-                        d2h(h_poff.data(), poff, n + 1, st);
-                        HIP_TRY(hipStreamSynchronize(st));
+                        down(h_poff.data(), poff, n + 1, st);
+                        settle(st);
                         if (mode_ == EngineMode::Record) plan_->poff.push_back(h_poff);
                     }
                     const uint64_t NB = h_poff[n];
@@ -1141,6 +1224,7 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
         }
     }
 
+    flush(st);
     t_child = ms_since(t_step);
     // ---- 4. finished runs, slot recycling, the new frontier ----
     for (auto* list : {&F_runs_, &next_runs})
@@ -1152,7 +1236,7 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
     std::vector<uint32_t> releasable;
     releasable.swap(release_next_);
     finalize(done_now);                        // synchronises the stream (not when capturing)
-    if (done_now.empty() && mode_ != EngineMode::Capture) HIP_TRY(hipStreamSynchronize(st));
+    if (done_now.empty() && mode_ != EngineMode::Capture) settle(st);
     t_fin = ms_since(t_step);
     prof_resolve(ctx_);
     for (uint32_t s : releasable) free_slots_.push_back(s);
@@ -1197,13 +1281,13 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
 // The exact (IR) hash and canonical edge ranks of a request's frontier states [b, e), computed
 // on the host from the generation's edges (the reference's device computes the same with its IR
 // canonicalizer when sampling, gpu/src/ir_canon.cu:152-280).
-void frontier_ir(const DevGen& G, uint32_t b, uint32_t e, hipStream_t st, RunRec& r) {
+void Engine::frontier_ir(const DevGen& G, uint32_t b, uint32_t e, hipStream_t st, RunRec& r) {
     const uint32_t n = e - b, A = G.v.A;
     std::vector<uint64_t> eo(n);
     std::vector<uint32_t> ne(n);
-    d2h(eo.data(), G.v.eoff + b, n, st);
-    d2h(ne.data(), G.v.ne + b, n, st);
-    HIP_TRY(hipStreamSynchronize(st));
+    down(eo.data(), G.v.eoff + b, n, st);
+    down(ne.data(), G.v.ne + b, n, st);
+    settle(st);
     uint64_t E = 0;
     for (uint32_t k = 0; k < n; ++k) E += ne[k];
     std::vector<uint8_t> ar(E);
@@ -1211,9 +1295,9 @@ void frontier_ir(const DevGen& G, uint32_t b, uint32_t e, hipStream_t st, RunRec
     // states of one request are contiguous in the generation, their edges too
     if (E) {
         const uint64_t e0 = eo[0];
-        d2h(ar.data(), G.v.ar + e0, E, st);
-        d2h(ev.data(), G.v.ev + e0 * A, E * A, st);
-        HIP_TRY(hipStreamSynchronize(st));
+        down(ar.data(), G.v.ar + e0, E, st);
+        down(ev.data(), G.v.ev + e0 * A, E * A, st);
+        settle(st);
     }
     std::vector<uint64_t> soff(n + 1, 0);
     std::vector<uint32_t> eoff(E + 1, 0), verts;
@@ -1247,12 +1331,12 @@ void Engine::sample_transitions(uint32_t n, uint32_t K, MatchView& mv, uint32_t*
     std::vector<uint32_t> rule(M0), cne(M0);
     std::vector<uint16_t> q(M0 * K);
     std::vector<uint64_t> off(n + 1);
-    d2h(h_parent.data(), mv.parent, M0, st);
-    d2h(rule.data(), mv.rule, M0, st);
-    d2h(q.data(), mv.q, M0 * K, st);
-    d2h(cne.data(), mv.cne, M0, st);
-    d2h(off.data(), moff, n + 1, st);
-    HIP_TRY(hipStreamSynchronize(st));
+    down(h_parent.data(), mv.parent, M0, st);
+    down(rule.data(), mv.rule, M0, st);
+    down(q.data(), mv.q, M0 * K, st);
+    down(cne.data(), mv.cne, M0, st);
+    down(off.data(), moff, n + 1, st);
+    settle(st);
     std::vector<uint8_t> keep(M0, 1);
     bool dropped = false;
     const uint32_t nF = (uint32_t)F_runs_.size();
@@ -1333,6 +1417,7 @@ void Engine::sample_transitions(uint32_t n, uint32_t K, MatchView& mv, uint32_t*
     up(mv.cne, cne2.data(), M1 + 1, st);
     up(cnt, cnt2.data(), n + 1, st);
     up(moff, off2.data(), n + 1, st);
+    flush(st);
     M = M1;
     mv.n = (uint32_t)M1;
     h_parent.swap(p2);
@@ -1358,8 +1443,8 @@ void Engine::sample_frontier(const std::vector<SampledKids>& kids, uint32_t nC, 
         const bool smp = !k.roots && S.frontier();
         if (smp && S.per_parent && h_parent.size() != M) {
             h_parent.resize(M);
-            d2h(h_parent.data(), mv.parent, M, st);
-            HIP_TRY(hipStreamSynchronize(st));
+            down(h_parent.data(), mv.parent, M, st);
+            settle(st);
         }
         uint64_t at_step = 0;
         std::unordered_map<uint32_t, uint64_t> at_parent;

@@ -16,6 +16,7 @@
 #include <string>
 #include <vector>
 
+#include "hgx_kernels.hpp"
 #include "hgx_runtime.hpp"
 
 namespace hgx {
@@ -187,6 +188,7 @@ private:
                             std::vector<uint32_t>& h_parent, hipStream_t st);
     // After a generation is built: which of the sampled requests' new states are expanded
     // (exploration coin, per-step and per-parent bounds, in event order), into F_expand_.
+    void frontier_ir(const DevGen& G, uint32_t b, uint32_t e, hipStream_t st, RunRec& r);
     void sample_frontier(const std::vector<SampledKids>& kids, uint32_t nC, const MatchView& mv, uint64_t M,
                          std::vector<uint32_t>& h_parent, hipStream_t st);
 
@@ -194,13 +196,34 @@ private:
     std::shared_ptr<PassPlan> plan_;
     size_t plan_rb_ = 0, plan_poff_ = 0;      // next plan entries (capture)
     uint32_t* d_check_ = nullptr;
-    std::vector<void*> pinned_;               // pinned staging of captured copies
+    std::vector<void*> pinned_;               // pinned staging of captured transfers
 
-    // Host-to-device copy of n elements: straight from src, or (capture) through pinned staging
-    // that lives as long as the engine, since a replay copies from it again.
+    // Small transfers between host and device, gathered: put() and get() stage each in pinned
+    // memory, flush() moves all of them in one launch (k_move), settle() flushes, waits for the
+    // stream and hands out what get() asked for. A copy by itself costs the runtime's staging and
+    // a launch of its own: a generation took 10 to 20 of them, 5 us each. Every put() is flushed
+    // before the launch that reads it. The staging is a lease of the context's pinned buffers, free
+    // again once the stream is idle (each step ends so); under capture it is the engine's own and
+    // lives as long, since a replay reads it again. Larger transfers, and those past the staging,
+    // are copies of their own.
+    static constexpr size_t kMoveMax = (size_t)256 << 10;
     void put(void* dst, const void* src, size_t bytes, hipStream_t st);
+    void get(void* dst, const void* src, size_t bytes, hipStream_t st);
+    void flush(hipStream_t st);
+    void settle(hipStream_t st);
+    uint8_t* stage(size_t bytes);             // staging for one transfer (null: none left)
+    void drop_moves();                        // forget what is staged (nothing in flight reads it)
+    struct Fetch { void* dst; const uint8_t* from; size_t bytes; };
+    std::shared_ptr<PinnedStage> stage_owner_;
+    std::unique_ptr<StageLease> lease_;
+    uint8_t* stage_p_ = nullptr;
+    size_t stage_used_ = 0, stage_size_ = 0;
+    std::vector<Move> moves_;
+    std::vector<Fetch> fetches_;
     template <class T>
     void up(T* dst, const T* src, size_t n, hipStream_t st) { put(dst, src, sizeof(T) * n, st); }
+    template <class T>
+    void down(T* dst, const T* src, size_t n, hipStream_t st) { get(dst, src, sizeof(T) * n, st); }
     void fill_counts(RunRec& r, const uint64_t* x);
 
     uint32_t step_impl(std::vector<std::shared_ptr<RunRec>>& admitted);

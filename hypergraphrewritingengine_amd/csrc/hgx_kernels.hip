@@ -1691,6 +1691,31 @@ __global__ void k_fill(uint8_t* p, uint32_t word, uint64_t words, uint64_t bytes
     if (i < bytes - words * 4) p[words * 4 + i] = (uint8_t)word;          // the tail bytes
 }
 
+// A workgroup per transfer, 16 bytes a thread where both ends allow it. Bound by the round trip to
+// host memory (4 us for a pass's two dozen transfers, which were a copy of 5 us each).
+__global__ __launch_bounds__(256) void k_move(const Move* moves) {
+    const Move m = moves[blockIdx.x];
+    static_assert(kMoveBytes == 16 * 256, "one 16-byte read per thread");
+    const uint64_t align = (uint64_t)m.dst | (uint64_t)m.src;
+    uint64_t done = 0;
+    if ((align & 15u) == 0) {
+        const uint64_t n = m.bytes / 16;
+        if (threadIdx.x < n) ((uint4*)m.dst)[threadIdx.x] = ((const uint4*)m.src)[threadIdx.x];
+        done = n * 16;
+    } else if ((align & 3u) == 0) {
+        const uint64_t n = m.bytes / 4;
+        for (uint64_t i = threadIdx.x; i < n; i += 256) ((uint32_t*)m.dst)[i] = ((const uint32_t*)m.src)[i];
+        done = n * 4;
+    }
+    for (uint64_t i = done + threadIdx.x; i < m.bytes; i += 256) ((uint8_t*)m.dst)[i] = ((const uint8_t*)m.src)[i];
+}
+
+hipError_t launch_move(const Move* moves, uint32_t n, hipStream_t st) {
+    if (!n) return hipSuccess;
+    hipLaunchKernelGGL(k_move, dim3(n), dim3(256), 0, st, moves);
+    return hipGetLastError();
+}
+
 hipError_t launch_fill(void* p, uint8_t value, uint64_t bytes, hipStream_t st) {
     if (!bytes) return hipSuccess;
     const uint32_t word = 0x01010101u * value;

@@ -238,6 +238,15 @@ hipError_t launch_mask_counts(const uint32_t* run, const uint8_t* active, uint32
 // Byte fill of [p, p + bytes) by a kernel: the engine clears its buffers with it (never
 // hipMemsetAsync), so a pass it records into a graph holds kernels and copies only.
 hipError_t launch_fill(void* p, uint8_t value, uint64_t bytes, hipStream_t st);
+// Transfers of at most kMoveBytes each between device and pinned host memory, n of them in one
+// launch; the list is in pinned memory too.
+constexpr uint64_t kMoveBytes = 4096;
+struct Move {
+    void* dst;
+    const void* src;
+    uint64_t bytes;
+};
+hipError_t launch_move(const Move* moves, uint32_t n, hipStream_t st);
 // A read-only launch of known traffic (bytes read, 8 written) for counter calibration.
 hipError_t launch_read_calibration(const void* p, uint64_t bytes, uint64_t* sink, hipStream_t st);
 hipError_t launch_read_gather(void* p, uint64_t bytes, uint64_t* sink, uint64_t* ctr, hipStream_t st);
