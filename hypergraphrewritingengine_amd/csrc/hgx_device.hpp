@@ -71,7 +71,8 @@ static_assert(offsetof(DRule, lv) % 4 == 0 && sizeof(DRule) % 4 == 0, "DRule is 
 struct DRun {
     const DRule* rules;      // this request's rules (device copy)
     uint32_t n_rules;
-    uint32_t n_roots, flags, pad0;
+    uint32_t n_roots, flags;
+    uint32_t count_lhs;      // branchial_rule_lhs() of its rules
     uint64_t* map_keys;      // open-addressing WL-hash set, first writer wins
     uint32_t map_mask;       // capacity - 1 (power of two)
     uint32_t zero_seen;      // the hash 0 is kept beside the table (0 is EMPTY)

@@ -238,6 +238,14 @@ void Engine::admit(std::shared_ptr<RunRec>& r) {
     d.n_rules = (uint32_t)r->hp->rules.size();
     d.n_roots = r->hp->n_roots();
     d.flags = r->hp->flags;
+    if (r->hp->rules.size() <= kBranchialRules) {
+        uint32_t most = 0, least = 0xFFFFFFFFu;
+        for (auto& R : r->hp->rules) {
+            most = std::max<uint32_t>(most, R.n_lhs);
+            least = std::min<uint32_t>(least, R.n_lhs);
+        }
+        if (most <= 3) d.count_lhs = most | (least == most ? 4u : 0u);
+    }
     d.map_keys = r->map_keys;
     d.map_mask = (uint32_t)(mc - 1);
     r->ne_bound = r->hp->max_root_ne;
@@ -1099,6 +1107,7 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
         std::vector<uint64_t> h_poff;
         if (M) {
             bool any_b = false, all_b = true, any_rel = false;
+            BranchialShape bsh{F_ ? F_->max_ne : 0u, false, false, 0, 0};
             std::vector<uint8_t> bflag(cap_slots_, 0);
             for (uint32_t i = 0; i < nF; ++i) {
                 if (!tot[i]) continue;
@@ -1107,6 +1116,11 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
                 bflag[r.slot] = b ? 1 : 0;
                 any_b |= b; all_b &= b;
                 any_rel |= b && (r.hp->flags & HGX_REC_RELATIONS);
+                if (!b) continue;
+                const uint32_t lhs = h_runs_[r.slot].count_lhs & 3u, t = (uint32_t)tot[i];
+                (lhs ? bsh.counted : bsh.rest) = true;
+                if (lhs) bsh.matches = std::max(bsh.matches, t);
+                if (lhs == 3) bsh.triples = std::max(bsh.triples, t);
             }
             if (any_b) {
                 uint32_t* bcnt = cnt;
@@ -1121,7 +1135,7 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
                 }
                 BranchialArgs ba{};
                 ba.P = F_->v; ba.M = mv; ba.runs = d_runs_; ba.cnt = bcnt; ba.moff = moff; ba.ctr = d_ctr_;
-                ba.emit = 0; ba.lds_per_wave = branchial_lds_per_wave();
+                ba.emit = 0;
                 uint32_t* pcnt = nullptr;
                 if (any_rel) {
                     pcnt = dalloc<uint32_t>(tmp, n + 1);
@@ -1129,7 +1143,7 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
                 }
                 ba.pcnt = pcnt;
                 timed(ctx_, st, "k_branchial", M * (6ull + 2ull * K) + n * 12ull, n,
-                      [&] { return launch_branchial(ba, ctx_->num_cu * 8, 2, st); });
+                      [&] { return launch_branchial(ba, bsh, ctx_->num_cu * 8, st); });
                 // parents above BR_MAX_EDGES edges: (edge slot, match) keys sorted into per-edge lists
                 BrListArgs bl{};
                 const bool large = F_->max_ne > BR_MAX_EDGES;
@@ -1179,7 +1193,7 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
                     if (NB) {
                         C->br_pairs = dalloc<uint32_t>(C->meta, 2 * NB);
                         ba.emit = 1; ba.poff = poff; ba.pairs = C->br_pairs;
-                        HIP_TRY(launch_branchial(ba, ctx_->num_cu * 8, 2, st));
+                        HIP_TRY(launch_branchial(ba, bsh, ctx_->num_cu * 8, st));
                         if (large) {
                             uint64_t* bo = dalloc<uint64_t>(tmp, M + 1);
                             scan_u32_to_u64(tmp, bl.bc, bo, (uint32_t)M, st);

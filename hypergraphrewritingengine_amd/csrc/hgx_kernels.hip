@@ -5,10 +5,11 @@
 //   k_match_bits     both over small binary states, by bit sets
 //   k_match_lists    both over larger binary states that fit the LDS, by lists per position
 //   k_expand         rewrite + WL hash, one team per child state
-//                    (k_expand_small: small children of one arity)
+//                    (k_expand_small, k_expand_large: children of one arity)
 //   k_record         each child's event, causal masks and records, its hash into its request's
 //                    state map, and the request's counters
-//   k_branchial      sibling-event overlap pairs, one wave per parent state (k_brl_*: the
+//   k_branchial      sibling-event overlap pairs, one wave per parent state (k_branchial_count:
+//                    only their number, where counters are cheaper than bit sets; k_brl_*: the
 //                    sorted per-edge lists for parents above 128 edges)
 //   k_wl_states      WL hash of given states (roots, and the hgx_wl_hash_batch entry point)
 //   small helpers    per-run totals, count masking, map rehash
@@ -354,7 +355,8 @@ constexpr uint64_t kNoBudget = 0xFFFFFFFFull;    // MatchArgs::budget of a run w
 // whose workspace would otherwise leave a CU one or two waves). The one-wave passes are held to
 // four waves per SIMD (128 registers): at five (96) the emit pass spilled 19 registers and 96
 // bytes per lane to scratch -- 25 MB of writes per launch instead of 3 MB -- and config 2 ran 3%
-// slower, while the batched pass times alike under both bounds.
+// slower, while the batched pass timed alike under both bounds (both measured on binary states, which
+// have kernels of their own now).
 // GWS: the workspace is a per-workgroup slice of global memory (a.scratch) -- the same code for
 // states too large for LDS, with W = 8. G < 64 (with W = 1): sub-wave teams, 64 / G states per
 // wave, each team with its own workspace, for small states whose seeds would leave most of a
@@ -1264,8 +1266,6 @@ hipError_t launch_match_lists(const MatchArgs& a, bool emit, uint32_t grid, uint
     const dim3 g(grid);
     const size_t lds = a.lds_per_wave;
     switch (team * 2 + (emit ? 1 : 0)) {
-        case 8: hipLaunchKernelGGL((k_match_lists<false, 4>), g, dim3(256), lds, st, a); break;
-        case 9: hipLaunchKernelGGL((k_match_lists<true, 4>), g, dim3(256), lds, st, a); break;
         case 16: hipLaunchKernelGGL((k_match_lists<false, 8>), g, dim3(512), lds, st, a); break;
         case 17: hipLaunchKernelGGL((k_match_lists<true, 8>), g, dim3(512), lds, st, a); break;
         case 32: hipLaunchKernelGGL((k_match_lists<false, 16>), g, dim3(1024), lds, st, a); break;
@@ -1317,8 +1317,9 @@ __device__ inline void wl_state_done(const WLStatesArgs& a, uint32_t i, uint64_t
 // team: W = 1, one wave per child (up to four per workgroup, each with its own workspace);
 // W > 1, the workgroup's W waves share one child and one workspace, for large children whose
 // workspace would otherwise leave a CU one or two waves. One-wave teams are held to four waves
-// per SIMD (128 registers, a few spilled): on the batched pass the expansion took 9.8 ms so,
-// 15.3 ms at three (no spill) and 11.1 ms at five (36 registers spilled).
+// per SIMD (about 100 registers, none spilled). When this kernel took the batched workload's
+// children too (k_expand_small does now), its expansion was 9.8 ms so, 15.3 ms at three waves and
+// 11.1 ms at five.
 template <bool GWS, uint32_t W, uint32_t G>
 __global__ __launch_bounds__(W == 1 ? 256 : 64 * W, W == 1 ? 4 : 1) void k_expand(ExpandArgs a) {
     using TM = typename TeamSel<W, G>::type;
@@ -2108,7 +2109,7 @@ hipError_t launch_record(const ExpandArgs& a, uint32_t n, hipStream_t st) {
 
 constexpr uint32_t BR_LDS_WORDS = 1024;             // per table: 8 KiB of bitsets, 8 KiB of masks
 
-uint32_t branchial_lds_per_wave() { return 2 * BR_LDS_WORDS * 8 + 64; }
+static uint32_t branchial_lds_per_wave() { return 2 * BR_LDS_WORDS * 8 + 64; }
 
 template <uint32_t NW>
 __device__ __forceinline__ void consumed_mask(const BranchialArgs& a, const DRun& RN, uint32_t m,
@@ -2219,6 +2220,144 @@ __device__ __forceinline__ uint32_t branchial_parent(const BranchialArgs& a, con
     return total;
 }
 
+// The pair counts of parents whose matches consume at most three edges, without the pairs. Two
+// matches of a parent that share k edges share k single edges, k (k - 1) / 2 edge pairs and, for
+// k = 3, one triple: single - pairs + triples is 1 for k = 1, 2 and 3. So each match adds itself to
+// a counter of each of its edges, of its edge pairs (a triangular table) and of its triple (a hash
+// table), and the counters' old values, with those signs, are the pairs it makes with earlier
+// matches: one pass over the matches, where the bit sets of k_branchial take one to build them and
+// one to read them for every 64 matches.
+// G lanes per parent: 16 for those of few edges in a generation of enough parents to fill the chip so
+// (bound by the latency of a parent's reads, so the parents in flight count), a wave for those of many
+// matches, whose time with bit sets grows as the square. Parents in between stay with k_branchial: the
+// tables of 65 to 128 edges take all the LDS of its bit sets (those of the batched workload's fifth
+// generation 0.23 ms by bit sets, 0.43 by a wave of counts each).
+// 300 k parents of one evolution 0.50 -> 0.06 ms; a generation with parents of up to 4,096 matches
+// 0.50 -> 0.07; the batched workload's counts 1.25 -> 0.84.
+__host__ __device__ inline uint32_t branchial_count_words(uint32_t ne) {
+    return ((ne + (ne * (ne - (ne ? 1u : 0u)) / 2 + 1) / 2) + 3u) & ~3u;
+}
+// Slots of the triples' table for cnt matches: a load of at most a half.
+__device__ __forceinline__ uint32_t branchial_slots(uint32_t cnt) {
+    uint32_t n = 32;
+    while (n < 2 * cnt) n <<= 1;
+    return n;
+}
+// Who counts a parent's pairs: 16 lanes (1), a wave (2) of k_branchial_count, or k_branchial (0).
+__device__ __forceinline__ uint32_t branchial_tier(const BranchialArgs& a, uint32_t count_lhs, uint32_t ne, uint32_t cnt) {
+    const uint32_t k = count_lhs & 3u;
+    if (k == 0) return 0;
+    if (ne <= a.few_ne && (k < 3 || cnt <= kBranchialFewTriples)) return 1;
+    return cnt > kBranchialMany && (k < 3 || cnt <= kBranchialTriples) ? 2 : 0;
+}
+template <uint32_t G>
+__device__ __forceinline__ uint32_t branchial_count(const BranchialArgs& a, const DRun& RN, uint32_t lhs, uint32_t* tab,
+                                                    uint32_t m0, uint32_t cnt, uint32_t ne, uint32_t r) {
+    const uint32_t words = branchial_count_words(ne), slots = (lhs & 3u) == 3 ? branchial_slots(cnt) : 0u;
+    uint32_t* triples = tab + words;
+    for (uint32_t i = r; i < (words + slots) / 4; i += G) ((uint4*)tab)[i] = make_uint4(0, 0, 0, 0);
+    wave_sync();
+    uint32_t pairs = 0;
+    auto edge_pair = [&](uint32_t x, uint32_t y) {
+        const uint32_t hi = x > y ? x : y, lo = x > y ? y : x, at = hi * (hi - 1) / 2 + lo, sh = 16 * (at & 1u);
+        pairs -= (atomicAdd(&tab[ne + at / 2], 1u << sh) >> sh) & 0xFFFFu;
+    };
+    for (uint32_t i = r; i < cnt; i += G) {
+        const uint32_t m = m0 + i;
+        const uint16_t* q = a.M.q + (size_t)m * a.M.K;
+        const uint32_t nl = lhs & 4u ? lhs & 3u : RN.rules[a.M.rule[m]].n_lhs;
+        const uint32_t x = q[0];
+        pairs += atomicAdd(&tab[x], 1u);
+        if (nl < 2) continue;
+        const uint32_t y = q[1];
+        pairs += atomicAdd(&tab[y], 1u);
+        edge_pair(x, y);
+        if (nl < 3) continue;
+        const uint32_t z = q[2];
+        pairs += atomicAdd(&tab[z], 1u);
+        edge_pair(x, z);
+        edge_pair(y, z);
+        const uint32_t lo = min(x, min(y, z)), hi = max(x, max(y, z));
+        const uint32_t key = (lo << 14 | (x + y + z - lo - hi) << 7 | hi) + 1;     // at most 22 bits
+        uint32_t h = (key * 0x9E3779B1u) >> 16 & (slots - 1);
+        for (;;) {                                     // (the table is at most half full)
+            const uint32_t was = atomicCAS(&triples[h], 0u, key << 10 | 1u);
+            if (was == 0) break;
+            if (was >> 10 == key) { pairs += atomicAdd(&triples[h], 1u) & 1023u; break; }
+            h = (h + 1) & (slots - 1);
+        }
+    }
+    wave_sync();
+    return group_sum<G>(pairs);
+}
+template <uint32_t G>
+__global__ __launch_bounds__(G == WAVE ? 64 : 256) void k_branchial_count(BranchialArgs a) {
+    extern __shared__ uint8_t lds[];
+    constexpr uint32_t GPW = WAVE / G, WPB = G == WAVE ? 1 : 4, SUMS = WPB * GPW;
+    __shared__ uint32_t srun[SUMS];
+    __shared__ uint64_t ssum[SUMS];
+    const uint32_t w = threadIdx.x / WAVE, l = lane_id(), g = l / G, r = l % G;
+    uint32_t* tab = (uint32_t*)(lds + (size_t)w * a.lds_per_wave) + g * a.group_words;
+    uint32_t cur = INV;                                // the run whose pairs `sum` holds
+    uint64_t sum = 0;
+    auto add = [&](uint32_t run, uint32_t total) {
+        if (run != cur) {
+            if (cur != INV && sum && r == 0)
+                atomicAdd((unsigned long long*)&a.ctr[(size_t)cur * CTR_N + CTR_BRANCHIAL], (unsigned long long)sum);
+            cur = run;
+            sum = 0;
+        }
+        sum += total;
+    };
+    // 16 lanes look at their parent; a wave, whose parents are rare, at 64 at a time (neighbours, which
+    // are often alike, to different waves), and takes those that are its own one by one
+    const uint64_t waves = (uint64_t)gridDim.x * WPB;
+    for (uint64_t base = (uint64_t)blockIdx.x * WPB + w; base * (WAVE / G) < a.P.n; base += G == WAVE ? waves * WAVE : waves) {
+        const uint64_t s = G == WAVE ? base + l * waves : base * GPW + g;
+        uint32_t cnt = 0, ne = 0, run = INV, m0 = 0, lhs = 0;
+        if (s < a.P.n) cnt = a.cnt[s];
+        if (cnt >= 2) {
+            ne = a.P.ne[s];
+            run = a.P.run[s];
+            m0 = (uint32_t)a.moff[s];
+            lhs = a.runs[run].count_lhs;
+        }
+        const bool live = cnt >= 2 && ne <= BR_MAX_EDGES && branchial_tier(a, lhs, ne, cnt) == (G == WAVE ? 2u : 1u);
+        if constexpr (G < WAVE) {
+            if (live) {
+                const uint32_t total = branchial_count<G>(a, a.runs[run], lhs, tab, m0, cnt, ne, r);
+                if (r == 0 && a.pcnt) a.pcnt[s] = total;
+                add(run, total);
+            }
+        } else {
+            for (uint64_t todo = __ballot(live); todo; todo &= todo - 1) {
+                const int at = __builtin_ctzll(todo);
+                auto of = [&](uint32_t v) { return (uint32_t)__builtin_amdgcn_readlane((int)v, at); };
+                const uint32_t one = of(run);
+                const uint32_t total = branchial_count<G>(a, a.runs[one], of(lhs), tab, of(m0), of(cnt), of(ne), r);
+                if (r == 0 && a.pcnt) a.pcnt[base + (uint64_t)at * waves] = total;
+                add(one, total);
+            }
+        }
+    }
+    // one add per workgroup and run (groups hold neighbouring parents, mostly one run's)
+    if (r == 0) { srun[w * GPW + g] = cur; ssum[w * GPW + g] = sum; }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t held = INV;
+        uint64_t t = 0;
+        for (uint32_t k = 0; k <= SUMS; ++k) {
+            if (k < SUMS && (srun[k] == INV || srun[k] == held)) {
+                if (srun[k] == held) t += ssum[k];
+                continue;
+            }
+            if (held != INV && t)
+                atomicAdd((unsigned long long*)&a.ctr[(size_t)held * CTR_N + CTR_BRANCHIAL], (unsigned long long)t);
+            if (k < SUMS) { held = srun[k]; t = ssum[k]; }
+        }
+    }
+}
+
 // The pairs of a run are added to its counter once per wave and run (a wave's states are mostly one
 // run's): an add per parent, 300 k of them to one evolution's counter, took 3.5 ms where the
 // counting itself takes 0.2.
@@ -2241,6 +2380,7 @@ __global__ __launch_bounds__(256) void k_branchial(BranchialArgs a) {
         const uint32_t run = a.P.run[s];
         const uint32_t m0 = (uint32_t)a.moff[s];
         const DRun& RN = a.runs[run];
+        if (!a.emit && branchial_tier(a, RN.count_lhs, ne, cnt)) continue;
         const uint32_t ev0 = RN.ev_base + (m0 - RN.child_begin);
         const uint64_t out = a.emit ? a.poff[s] : 0;
         const uint32_t total = ne <= 64 ? branchial_parent<1>(a, RN, m0, cnt, ne, ev0, out, my, l)
@@ -2554,10 +2694,29 @@ hipError_t launch_expand(const ExpandArgs& a, uint32_t grid_cap, uint32_t wpb, u
     return hipGetLastError();
 }
 
-hipError_t launch_branchial(const BranchialArgs& a, uint32_t grid_cap, uint32_t wpb, hipStream_t st) {
-    const uint32_t grid = grid_for(a.P.n, wpb, grid_cap);
-    const size_t lds = (size_t)a.lds_per_wave * wpb;
-    hipLaunchKernelGGL(k_branchial, dim3(grid), dim3(64 * wpb), lds, st, a);
+hipError_t launch_branchial(BranchialArgs a, const BranchialShape& h, uint32_t grid_cap, hipStream_t st) {
+    const uint32_t most = h.max_ne < BR_MAX_EDGES ? h.max_ne : BR_MAX_EDGES;
+    a.few_ne = 0;
+    if (!a.emit && h.counted) {
+        if (a.P.n >= kBranchialQuarter) {
+            a.few_ne = most < kBranchialFewEdges ? most : kBranchialFewEdges;
+            a.group_words = branchial_count_words(a.few_ne) + (h.triples ? 2 * kBranchialFewTriples : 0u);
+            a.lds_per_wave = 16 * a.group_words;
+            hipLaunchKernelGGL(k_branchial_count<16>, dim3(grid_for(a.P.n, 16, grid_cap)), dim3(256),
+                               (size_t)a.lds_per_wave * 4, st, a);
+            if (most <= a.few_ne && !h.rest && !h.triples) return hipGetLastError();
+        }
+        if (h.matches > kBranchialMany) {
+            uint32_t cnt = 0;                          // matches of the largest parent with triples
+            if (h.triples) for (cnt = 16; cnt < h.triples && cnt < kBranchialTriples;) cnt <<= 1;
+            a.group_words = branchial_count_words(most) + 2 * cnt;
+            a.lds_per_wave = 4 * a.group_words;
+            hipLaunchKernelGGL(k_branchial_count<64>, dim3(grid_for(a.P.n, 1, grid_cap)), dim3(64),
+                               a.lds_per_wave, st, a);
+        }
+    }
+    a.lds_per_wave = branchial_lds_per_wave();
+    hipLaunchKernelGGL(k_branchial, dim3(grid_for(a.P.n, 2, grid_cap)), dim3(128), (size_t)a.lds_per_wave * 2, st, a);
     return hipGetLastError();
 }
 

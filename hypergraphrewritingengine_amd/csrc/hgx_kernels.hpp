@@ -102,7 +102,9 @@ struct BranchialArgs {
     uint32_t* pcnt;            // [P.n] pairs per parent (may be null in count mode)
     const uint64_t* poff;      // [P.n + 1] exclusive offsets (emit)
     uint32_t* pairs;           // [2 * total] event ids within the run
-    uint32_t lds_per_wave;     // branchial_lds_per_wave()
+    // set by launch_branchial: LDS per wave and (counts) per parent, and the edges of the parents 16
+    // lanes take (0: none)
+    uint32_t lds_per_wave, group_words, few_ne;
 };
 
 // Branchial pairs of parents above 64 edges (per-edge lists of consuming matches).
@@ -217,11 +219,25 @@ uint32_t expand_grid(uint32_t n_items, uint32_t team, uint32_t wpb, uint32_t gri
 hipError_t launch_record(const ExpandArgs& a, uint32_t n, hipStream_t st);
 // grid used by the launchers for `items` work items (for sizing global scratch)
 uint32_t launch_grid(uint32_t items, uint32_t wpb, uint32_t grid_cap);
-uint32_t branchial_lds_per_wave();
 // Parents above this many edges have their branchial pairs found through sorted per-edge match
 // lists (launch_brl); smaller ones through LDS bitsets (launch_branchial).
 constexpr uint32_t BR_MAX_EDGES = 128;
-hipError_t launch_branchial(const BranchialArgs& a, uint32_t grid_cap, uint32_t wpb, hipStream_t st);
+// Counts without pairs (emit 0) for the requests whose rules have at most three LHS edges each:
+// count_lhs, else 0, is the largest of them (bits 0-1) and whether they are all as large (bit 2). A
+// request has at most kBranchialRules rules then, since the matches with the same three edges, six per
+// rule, are counted in 10 bits. By 16 lanes in generations of at least kBranchialQuarter parents, for
+// parents of at most kBranchialFewEdges edges (and with three LHS edges kBranchialFewTriples matches);
+// by a wave above kBranchialMany matches (with three LHS edges up to kBranchialTriples, 32 KB of table).
+constexpr uint32_t kBranchialRules = 170;
+constexpr uint32_t kBranchialQuarter = 16384;
+constexpr uint32_t kBranchialFewEdges = 48, kBranchialFewTriples = 64;
+constexpr uint32_t kBranchialMany = 512, kBranchialTriples = 4096;
+struct BranchialShape {
+    uint32_t max_ne;           // edges of the largest parent
+    bool counted, rest;        // some request, or not every one, has count_lhs
+    uint32_t matches, triples; // the most matches of a request with count_lhs, and with three LHS edges
+};
+hipError_t launch_branchial(BranchialArgs a, const BranchialShape& h, uint32_t grid_cap, hipStream_t st);
 uint32_t wl_states_lds_per_wave(uint32_t max_ne, uint32_t max_nv, uint32_t A, bool lean);
 // team: waves per state (1, 2, 4 or 8); with team 1, wpb states per workgroup.
 hipError_t launch_wl_states(const WLStatesArgs& a, uint32_t grid_cap, uint32_t wpb, uint32_t team, hipStream_t st);

@@ -6,7 +6,8 @@
 // waves per state, the lanes per state when one wave is the team (16 / 32 / 64), and the
 // workgroups per CU. Each candidate is run over a caller's prepared batch with the
 // launches event-timed per class, and each class keeps the fastest candidate (classes are separate
-// launches, so one sweep serves them all). The choice is kept in the context and written to a JSON
+// launches, so one sweep serves them all). Children of one arity and binary states take kernels whose
+// shapes follow from their sizes; the tuned shapes are those of the general kernels. The choice is kept in the context and written to a JSON
 // cache keyed by "<arch>:<CUs>", which hgx_ctx_create loads for its device (from HGX_TUNE_CACHE,
 // else tune_cache.json beside the library). None of the shapes changes a result -- the tests run
 // every lane count and team size against the oracle. The join order is not tuned: event numbering

@@ -200,19 +200,22 @@ size_t hgx_device_info(const hgx_ctx* ctx, char* buf, size_t len);
  *   HGX_OPTION_FORWARD  incremental match forwarding for states made by the previous
  *                       generation (ParallelEvolutionEngine's forwarding, enabled there by
  *                       rule_analysis forwarding_pays, hypergraph/src/rule_analysis.cpp:134):
- *                       1 on, 0 off (full join for every state), -1 automatic (default).
+ *                       1 on, 0 off (full join for every state), -1 automatic (default: states
+ *                       above 512 edges whose full join does not fit the device's LDS kernels).
  *   HGX_OPTION_DELTA_CAP delta matches one forwarded state may stage on chip, 1..4096
  *                       (default 256); a state with more takes the full join.
  *   HGX_OPTION_EXPAND_TEAM waves that rewrite and hash one child: 1, 2, 4 or 8 for every
- *                       child, 0 automatic (default: one wave for children whose workspace is
+ *                       child, 0 automatic (default: children of one arity by size, down to 8 lanes
+ *                       each and up to 16 waves; others one wave for children whose workspace is
  *                       small, a workgroup of 4 or 8 waves sharing one workspace for large ones).
  *   HGX_OPTION_JOIN_TEAM waves that join one parent state: 1, 4 or 8 for every state, 0 automatic
- *                       (chosen the same way).
+ *                       (chosen the same way; binary states by bit sets, 16 lanes each, or by lists,
+ *                       8 or 16 waves each).
  *   HGX_OPTION_EXPAND_LANES lanes that rewrite and hash one child when one wave is the team:
  *                       64, or 32 / 16 (sub-wave teams: two or four children per wave, each in
  *                       its own workspace), for every size class whose wave workspaces fit a
- *                       workgroup's LDS; 0 automatic (default: 16 lanes for children of up to 32
- *                       edges, 32 up to 64, else 64).
+ *                       workgroup's LDS; 0 automatic (default: children of one arity 16 lanes up to
+ *                       64 edges, 32 up to 128, else 64; others the tuned or default shape).
  *   HGX_OPTION_JOIN_LANES lanes that join one parent state when one wave is the team: 64, or
  *                       32 / 16 (two or four states per wave, each in its own workspace); 0
  *                       automatic (the tuned or default shape per size class).
