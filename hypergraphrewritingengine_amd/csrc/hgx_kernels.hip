@@ -54,6 +54,21 @@ __device__ inline uint32_t xcd_block() {
 //           enumerates, so event numbering is identical across engines and runs.
 // ------------------------------------------------------------------------------------------
 
+// Counts. A state's matches, a round's and a run's tally are added in 64 bits, and a state stops being
+// counted once it passes what its run may still take -- its cap or, without one, the 2^32 - 1 a count
+// holds: the run's generation is then refused whatever the other states hold. A seed is given up at
+// kSeedMany (the last depth adds at most 65,535 between two looks) and stands for 2^32.
+constexpr uint64_t kNoBudget = 0xFFFFFFFFull;     // MatchArgs::budget of a run without a cap
+constexpr uint32_t kSeedMany = 0xFFFE0000u;
+// Without a cap only counts above this are added to the run's tally: the adds of one run's 300 k states
+// to one word took 4 ms, and the few that matter for 2^32 are large.
+constexpr uint64_t kTallyMany = 4096;
+__device__ __forceinline__ uint64_t seed_count(uint32_t c) { return c < kSeedMany ? c : kNoBudget + 1; }
+__device__ __forceinline__ uint32_t stored_count(uint64_t n) { return n < kNoBudget ? (uint32_t)n : (uint32_t)kNoBudget; }
+__device__ __forceinline__ void add_tally(const MatchArgs& a, uint32_t run, bool capped, uint64_t n) {
+    if (capped ? n != 0 : n > kTallyMany) atomicAdd(&a.run_acc[run], (unsigned long long)n);
+}
+
 // Per-lane depth-first state: the edge bound at each depth, the bound-variable mask on entry to
 // each depth, the next candidate and the end of the candidate range at each depth, and the
 // variable bindings. Rules up to 16 LHS edges and variable ids up to 31 keep it per lane in
@@ -156,7 +171,7 @@ __device__ __forceinline__ uint32_t join_seed(const DRule& R, const uint32_t* sv
                     for (uint32_t t = 0; t < n; ++t) q_out[o * K + R.order[t]] = (uint16_t)L.matched[t];
                     par_out[o] = parent; rule_out[o] = rule_id; cne_out[o] = child_ne;
                 }
-                ++found;
+                if (++found == kSeedMany && !q_out) return found;
                 continue;
             }
             L.smask[d + 1] = m;
@@ -236,7 +251,7 @@ __device__ __forceinline__ uint32_t join_anchor(const DRule& R, uint32_t p, cons
                     o[0] = (uint16_t)rule_id;
                     for (uint32_t t = 0; t < n; ++t) o[1 + ord[t]] = (uint16_t)L.matched[t];
                 }
-                ++found;
+                if (++found == kSeedMany && !d_out) return found;
                 continue;
             }
             L.smask[d + 1] = m;
@@ -308,6 +323,7 @@ __device__ __forceinline__ uint32_t reg_join(const DRule& R, const uint32_t* sv,
             if (!ok) continue;
             m[D] = e;
             found = reg_join<N, D + 1, OUT>(R, sv, sa, ne, A, iend, ie, m, o, found);
+            if (!OUT && D + 1 < N && found >= kSeedMany) return found;   // (the last depth adds at most 65,535)
         }
         return found;
     }
@@ -347,8 +363,6 @@ uint32_t match_lds_per_wave(uint32_t max_ne, uint32_t max_nextv, uint32_t A, uin
     if (dmax) b += al(dmax * (KL + 1) * 2) + al(dmax * 2) + al((dmax + 1) * 4);
     return b;
 }
-
-constexpr uint64_t kNoBudget = 0xFFFFFFFFull;    // MatchArgs::budget of a run without a cap
 
 // W is the team: one wave per state (W = 1, up to four per workgroup, each with its own
 // workspace) or the W waves of a workgroup sharing one state and one workspace (large states,
@@ -431,10 +445,9 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W, W == 1 ? 4 : 1) void k_match
         const uint32_t nvid = a.P.nextv[s];                     // labels are < nvid
         const uint8_t active = a.active[run] && (!a.smask || a.smask[s]);
         const uint64_t budget = EMIT ? 0 : (uint64_t)a.budget[run];
-        // the run's tally moves under other teams: one read, shared, so the team agrees. A run without
-        // a cap keeps none: the adds of one run's 300 k states to one word took 4 ms.
-        const bool capped = !EMIT && budget != kNoBudget;
-        const uint64_t tally = capped ? tm.bcast(tm.leader() ? (uint64_t)a.run_acc[run] : 0ull) : 0ull;
+        // the run's tally moves under other teams: one read, shared, so the team agrees
+        const bool capped = budget != kNoBudget;
+        const uint64_t tally = EMIT ? 0 : tm.bcast(tm.leader() ? (uint64_t)a.run_acc[run] : 0ull);
         if (!active || (!EMIT && tally > budget)) {
             if (!EMIT && tm.leader()) { a.cnt[s] = 0; a.state_edges[s] = 0; }
             continue;
@@ -503,7 +516,7 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W, W == 1 ? 4 : 1) void k_match
         } else {
             rules = RN.rules;
         }
-        uint32_t total = 0;
+        uint64_t total = 0;
         uint64_t edges_sum = 0;                                // count pass: edges of the children
         bool stop = false;
         uint32_t out = EMIT ? (uint32_t)a.moff[s] : 0u;
@@ -526,7 +539,7 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W, W == 1 ? 4 : 1) void k_match
                 pp = i / nprod;
                 j = i % nprod;
             };
-            uint32_t nd = 0;
+            uint64_t nd = 0;
             uint64_t de = 0;                                    // child edges of the delta matches
             for (uint32_t base = 0; base < ncombo; base += N) {
                 const uint32_t i = base + tm.r;
@@ -537,7 +550,7 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W, W == 1 ? 4 : 1) void k_match
                     c = join_anchor(rules[r], pp, sv, sa, ne, A, iend, il, kept, kept + j, L, nullptr, 0, 0);
                     de += (uint64_t)c * (ne - rules[r].n_lhs + rules[r].n_rhs);
                 }
-                nd += tm.sum(c);
+                nd += tm.sum64(seed_count(c));
             }
             if (!EMIT || (a.dmax && nd <= a.dmax)) {
                 full = false;
@@ -626,7 +639,7 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W, W == 1 ? 4 : 1) void k_match
                 } else {
                     total = nf + nd;
                     edges_sum = tm.sum64(de);
-                    if (tm.leader() && total && capped) atomicAdd(&a.run_acc[run], (unsigned long long)total);
+                    if (tm.leader()) add_tally(a, run, capped, total);
                 }
             }
         }
@@ -692,13 +705,12 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W, W == 1 ? 4 : 1) void k_match
                     // The run's shared tally: once it passes what the run may still take, the
                     // generation is over the cap whatever the other states hold, so stop. Every
                     // state's count equals what it added, so the totals stay over the cap.
-                    const uint32_t round = tm.sum(c);
+                    const uint64_t round = tm.sum64(seed_count(c));
                     total += round;
-                    edges_sum += (uint64_t)round * child_ne;
-                    if (!capped) {
-                    } else if (base + N >= nseed && r + 1 >= RN.n_rules) {
-                        // the state's last round: nothing is left to stop, so add without waiting
-                        if (tm.leader() && round) atomicAdd(&a.run_acc[run], (unsigned long long)round);
+                    edges_sum += round * child_ne;
+                    if ((base + N >= nseed && r + 1 >= RN.n_rules) || (!capped && total <= kTallyMany)) {
+                        // the state's last round, or one not worth it: nothing to stop, no wait
+                        if (tm.leader()) add_tally(a, run, capped, round);
                     } else {
                         unsigned long long before = 0;
                         if (tm.leader() && round) before = atomicAdd(&a.run_acc[run], (unsigned long long)round);
@@ -710,7 +722,7 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W, W == 1 ? 4 : 1) void k_match
             tm.sync();
         }
         if (!EMIT && tm.leader()) {
-            a.cnt[s] = total;
+            a.cnt[s] = stored_count(total);
             a.state_edges[s] = edges_sum;
         }
     }
@@ -877,8 +889,7 @@ __global__ __launch_bounds__(256) void k_match_bits(MatchArgs a) {
         const uint32_t nm = EMIT ? a.cnt[s] : 0u;
         const uint8_t active = a.active[run] && (!a.smask || a.smask[s]);
         const uint64_t budget = EMIT ? 0 : (uint64_t)a.budget[run];
-        const bool capped = !EMIT && budget != kNoBudget;
-        const uint64_t tally = capped ? tm.bcast(tm.leader() ? (uint64_t)a.run_acc[run] : 0ull) : 0ull;
+        const uint64_t tally = EMIT ? 0 : tm.bcast(tm.leader() ? (uint64_t)a.run_acc[run] : 0ull);
         if (!active || (EMIT ? nm == 0 : tally > budget)) {
             if (!EMIT && tm.leader()) { a.cnt[s] = 0; a.state_edges[s] = 0; }
             continue;
@@ -912,15 +923,19 @@ __global__ __launch_bounds__(256) void k_match_bits(MatchArgs a) {
                 if ((base >> 6) == k) J.loops.w[k] |= lb;
         }
         tm.sync();
-        uint32_t total = 0;
+        const uint64_t room = budget - tally;                  // count pass: matches the run may still take
+        uint64_t total = 0;
         uint64_t edges_sum = 0;                                // count pass: edges of the children
         uint32_t out = EMIT ? (uint32_t)a.moff[s] : 0u;
-        for (uint32_t r = 0; r < n_rules; ++r) {
+        for (uint32_t r = 0; r < n_rules && (EMIT || total <= room); ++r) {
             const DRule& R = rules[r];
             if (!R.bits_ok) continue;                           // a pattern edge that is not binary
             const uint32_t n_lhs = R.n_lhs, child_ne = ne - n_lhs + R.n_rhs;
 #pragma unroll
             for (int d = 0; d < 4; ++d) J.bj[d] = R.bj[d];
+            // one rule's matches fit 32 bits (255 * 254 * 253 * 252); a sum past what is left has one
+            // lane past its share, so the sum is formed only then
+            const uint32_t left = (uint32_t)(room - total), share = left / N;
             uint32_t mine = 0;
             for (uint32_t base = 0; base < ne; base += N) {
                 const uint32_t seed = base + tm.r;
@@ -928,7 +943,7 @@ __global__ __launch_bounds__(256) void k_match_bits(MatchArgs a) {
                 const bool ok = seed < ne && (!(J.bj[0] & 256u) || (sv & 0xFFu) == sv >> 8);
                 const uint32_t c = ok ? bit_join_any<NW, false>(J, n_lhs, seed, sv, RegJoinOut{}) : 0u;
                 mine += c;
-                if (capped && mine > budget) break;            // (count pass) the run is over its cap
+                if (!EMIT && tm.any(mine > share) && tm.sum(mine) > left) break;
                 if constexpr (EMIT) {
                     uint32_t round;
                     const uint32_t inc = tm.incl_scan(c, round);
@@ -946,10 +961,10 @@ __global__ __launch_bounds__(256) void k_match_bits(MatchArgs a) {
             }
         }
         if (!EMIT && tm.leader()) {
-            a.cnt[s] = total;
+            a.cnt[s] = stored_count(total);
             a.state_edges[s] = edges_sum;
             // the run's shared tally: past what the run may still take its other states are skipped
-            if (total && capped) atomicAdd(&a.run_acc[run], (unsigned long long)total);
+            add_tally(a, run, budget != kNoBudget, total);
         }
     }
 }
@@ -1002,10 +1017,16 @@ struct ListJoin {
     const uint16_t* l1;
     uint32_t ne;
     uint32_t bj[4];
+    uint64_t most;             // count pass: a seed with more matches is given up
 };
 
+// Matches of a seed: a hub's pass 32 bits from four pattern edges on; one that is written fits.
+template <bool OUT>
+using ListCount = std::conditional_t<OUT, uint32_t, uint64_t>;
+
 template <int N, int D, bool OUT>
-__device__ __forceinline__ uint32_t list_join(const ListJoin& J, Bound B, const RegJoinOut& o, uint32_t found) {
+__device__ __forceinline__ ListCount<OUT> list_join(const ListJoin& J, Bound B, const RegJoinOut& o,
+                                                    ListCount<OUT> found) {
     if constexpr (D == N) {
         if constexpr (OUT) {
             const size_t at = (size_t)(o.base + found);
@@ -1061,14 +1082,15 @@ __device__ __forceinline__ uint32_t list_join(const ListJoin& J, Bound B, const 
             if (!ok) continue;
             B.template set<D>(e, v);
             found = list_join<N, D + 1, OUT>(J, B, o, found);
+            if (!OUT && D + 1 < N && found > J.most) return found;
         }
         return found;
     }
 }
 
 template <bool OUT>
-__device__ __forceinline__ uint32_t list_join_any(const ListJoin& J, uint32_t n_lhs, uint32_t seed, uint32_t sv,
-                                                  const RegJoinOut& o) {
+__device__ __forceinline__ ListCount<OUT> list_join_any(const ListJoin& J, uint32_t n_lhs, uint32_t seed, uint32_t sv,
+                                                        const RegJoinOut& o) {
     const Bound B{seed, 0, 0, 0, sv, 0, 0, 0};
     switch (n_lhs) {
         case 1: return list_join<1, 1, OUT>(J, B, o, 0u);
@@ -1148,9 +1170,8 @@ __global__ __launch_bounds__(64 * W) void k_match_lists(MatchArgs a) {
         const uint32_t nvid = a.P.nextv[s];                     // labels are < nvid
         const uint8_t active = a.active[run] && (!a.smask || a.smask[s]);
         const uint64_t budget = EMIT ? 0 : (uint64_t)a.budget[run];
-        const bool capped = !EMIT && budget != kNoBudget;
         // one read of the run's tally, which moves under other workgroups, for all of the team
-        const uint64_t tally = capped ? tm.bcast(l == 0 ? (uint64_t)a.run_acc[run] : 0ull) : 0ull;
+        const uint64_t tally = EMIT ? 0 : tm.bcast(l == 0 ? (uint64_t)a.run_acc[run] : 0ull);
         if (!active || (EMIT ? a.cnt[s] == 0 : tally > budget)) {
             if (!EMIT && l == 0) { a.cnt[s] = 0; a.state_edges[s] = 0; }
             continue;
@@ -1214,43 +1235,48 @@ __global__ __launch_bounds__(64 * W) void k_match_lists(MatchArgs a) {
         const DRun& RN = a.runs[run];
         ListJoin J;
         J.ev = ev; J.end = end; J.l0 = l0; J.l1 = l1; J.ne = ne;
-        uint32_t total = 0;
+        const uint64_t room = budget - tally;                  // count pass: matches the run may still take
+        uint64_t total = 0;
         uint64_t edges_sum = 0;                                // count pass: edges of the children
         uint32_t out = EMIT ? (uint32_t)a.moff[s] : 0u;
-        for (uint32_t r = 0; r < RN.n_rules; ++r) {
+        for (uint32_t r = 0; r < RN.n_rules && (EMIT || total <= room); ++r) {
             const DRule& R = RN.rules[r];
             if (!R.bits_ok) continue;                           // a pattern edge that is not binary
             const uint32_t n_lhs = R.n_lhs, child_ne = ne - n_lhs + R.n_rhs;
 #pragma unroll
             for (int d = 0; d < 4; ++d) J.bj[d] = R.bj[d];
-            uint32_t mine = 0;
+            const uint64_t left = room - total;
+            uint64_t mine = 0;
+            J.most = EMIT ? kNoBudget : left;
             for (uint32_t base = 0; base < ne; base += N) {
                 const uint32_t seed = base + l;
                 const uint32_t sv = seed < ne ? ev[seed] : 0u;
                 const bool ok = seed < ne && (!(J.bj[0] & 256u) || (sv & 0xFFFFu) == sv >> 16);
-                const uint32_t c = ok ? list_join_any<false>(J, n_lhs, seed, sv, RegJoinOut{}) : 0u;
+                const uint64_t c = ok ? list_join_any<false>(J, n_lhs, seed, sv, RegJoinOut{}) : 0u;
                 mine += c;
-                if (capped && mine > budget) break;            // (count pass) the run is over its cap
+                // a sum past what is left has one lane past its share
+                if (!EMIT && base + N < ne && tm.any(mine > left / N) && tm.sum64(mine) > left) break;
                 if constexpr (EMIT) {
                     uint32_t round;
-                    const uint32_t inc = tm.incl_scan(c, round);
+                    const uint32_t inc = tm.incl_scan((uint32_t)c, round);
                     if (c) {
-                        const RegJoinOut ro{a.M.q, a.M.K, out + inc - c, a.M.parent, a.M.rule, a.M.cne, s, r, child_ne};
+                        const RegJoinOut ro{a.M.q, a.M.K, out + inc - (uint32_t)c, a.M.parent, a.M.rule, a.M.cne, s, r,
+                                            child_ne};
                         list_join_any<true>(J, n_lhs, seed, sv, ro);
                     }
                     out += round;
                 }
             }
             if constexpr (!EMIT) {
-                const uint32_t sum = tm.sum(mine);
+                const uint64_t sum = tm.sum64(mine);
                 total += sum;
-                edges_sum += (uint64_t)sum * child_ne;
+                edges_sum += sum * child_ne;
             }
         }
         if (!EMIT && l == 0) {
-            a.cnt[s] = total;
+            a.cnt[s] = stored_count(total);
             a.state_edges[s] = edges_sum;
-            if (total && capped) atomicAdd(&a.run_acc[run], (unsigned long long)total);
+            add_tally(a, run, budget != kNoBudget, total);
         }
     }
 }
