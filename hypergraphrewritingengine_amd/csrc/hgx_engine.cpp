@@ -549,27 +549,34 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
             ma.run_acc = (unsigned long long*)d_run_acc_;
             ma.state_edges = dalloc<uint64_t>(tmp, n);
             const uint64_t match_bytes = F_->n_edges * (4ull * F_->v.A + 1) + (uint64_t)n * 24;
-            // One launch per size class of the requests taking part (by their bound on state
-            // edges), each with LDS staging sized for its class; states outside the launches
-            // (requests not advancing) keep the zero count set here.
+            // The size class of each request taking part, by its bound on state edges; few states of
+            // up to 128 edges are one class, as for the children. Decided once for both passes: the
+            // emit pass of a class leaves out the requests that stopped between them, so whatever
+            // kernel emits a class counted it too, and reads what that count left (seedcnt).
+            std::vector<int> jcls(nF, -1);
+            {
+                uint64_t n_small = 0;
+                for (uint32_t i = 0; i < nF; ++i)
+                    if (h_active[F_runs_[i]->slot] && F_runs_[i]->ne_bound <= kClassEdges[kMergeClass])
+                        n_small += F_e_[i] - F_b_[i];
+                for (uint32_t i = 0; i < nF; ++i) {
+                    const RunRec& r = *F_runs_[i];
+                    if (!h_active[r.slot] || F_e_[i] == F_b_[i]) continue;
+                    int k = 0;
+                    while (r.ne_bound > kClassEdges[k]) ++k;
+                    if (n_small < kMergeBelow && k < kMergeClass) k = kMergeClass;
+                    jcls[i] = k;
+                }
+            }
+            // One launch per size class, each with LDS staging sized for its class; states outside
+            // the launches (requests not advancing) keep the zero count set here.
             auto launch_classes = [&](bool emit, std::vector<ExpandClass>& cls, const char* name,
                                       uint64_t bytes) {
                 cls.assign(6, ExpandClass{});
-                // few states of up to 128 edges: one class of them all, as for the children
-                uint64_t n_small = 0;
-                for (uint32_t i = 0; i < nF; ++i)
-                    if ((emit ? tot[i] != 0 : h_active[F_runs_[i]->slot] != 0) &&
-                        F_runs_[i]->ne_bound <= kClassEdges[kMergeClass])
-                        n_small += F_e_[i] - F_b_[i];
-                const bool merge = n_small < kMergeBelow;
                 for (uint32_t i = 0; i < nF; ++i) {
                     const RunRec& r = *F_runs_[i];
-                    if (emit ? !tot[i] : !h_active[r.slot]) continue;
-                    if (F_e_[i] == F_b_[i]) continue;
-                    int k = 0;
-                    while (r.ne_bound > kClassEdges[k]) ++k;
-                    if (merge && k < kMergeClass) k = kMergeClass;
-                    ExpandClass& x = cls[k];
+                    if (jcls[i] < 0 || (emit && !tot[i])) continue;
+                    ExpandClass& x = cls[jcls[i]];
                     x.ne = std::max(x.ne, r.ne_bound);
                     x.nextv = std::max(x.nextv, r.nv_bound);
                     x.uniform = x.uniform && r.hp->bits_join;
