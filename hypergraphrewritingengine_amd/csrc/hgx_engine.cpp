@@ -988,7 +988,9 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
                 if (x.n != M) {
                     ea.rb = x.d_rb; ea.rpre = x.d_rb + x.rb.size(); ea.nrange = (uint32_t)x.rb.size();
                 }
-                if (ea.lean && ea.max_child_ne <= kSmallMaxEdges && ea.max_nextv <= kSmallMaxLabels &&
+                // (a request of arity 5 and up in another class widens the generation's edges past
+                // both one-arity kernels)
+                if (ea.lean && A <= 4 && ea.max_child_ne <= kSmallMaxEdges && ea.max_nextv <= kSmallMaxLabels &&
                     ctx_->expand_team <= 1) {
                     const SmallShape sh = small_shape(ea, K, ctx_->expand_lanes, ctx_->max_lds, A);
                     ea.lds_per_wave = sh.lds;
