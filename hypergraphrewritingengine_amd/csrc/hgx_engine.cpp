@@ -609,7 +609,7 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
                     // lanes per state (batched count pass 0.85 ms, 1.04 with 32; few states time
                     // alike), up to 32 workgroups per CU (0.94 ms at 8, 0.86 at 16).
                     const uint32_t nw = match_bits_words(mc.max_ne);
-                    if (x.uniform && nw && mc.max_nextv <= kMatchBitsLabels && !mc.fwd_n && ctx_->join_team <= 1) {
+                    if (x.uniform && nw && mc.max_nextv <= kMatchBitsLabels && !mc.fwd_n && !ctx_->join_team) {
                         mc.lds_per_wave = match_bits_lds(mc.max_ne, mc.max_nextv, nw);
                         uint32_t lanes = ctx_->join_lanes ? ctx_->join_lanes : 16u;
                         while (lanes < 64 && (uint64_t)mc.lds_per_wave * (64 / lanes) > ctx_->max_lds) lanes *= 2;
@@ -991,7 +991,7 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
                 // (a request of arity 5 and up in another class widens the generation's edges past
                 // both one-arity kernels)
                 if (ea.lean && A <= 4 && ea.max_child_ne <= kSmallMaxEdges && ea.max_nextv <= kSmallMaxLabels &&
-                    ctx_->expand_team <= 1) {
+                    !ctx_->expand_team) {
                     const SmallShape sh = small_shape(ea, K, ctx_->expand_lanes, ctx_->max_lds, A);
                     ea.lds_per_wave = sh.lds;
                     timed(ctx_, st, "k_expand", (uint64_t)((double)bytes * x.n / M), x.n,

@@ -205,12 +205,14 @@ size_t hgx_device_info(const hgx_ctx* ctx, char* buf, size_t len);
  *   HGX_OPTION_DELTA_CAP delta matches one forwarded state may stage on chip, 1..4096
  *                       (default 256); a state with more takes the full join.
  *   HGX_OPTION_EXPAND_TEAM waves that rewrite and hash one child: 1, 2, 4 or 8 for every
- *                       child, 0 automatic (default: children of one arity by size, down to 8 lanes
- *                       each and up to 16 waves; others one wave for children whose workspace is
- *                       small, a workgroup of 4 or 8 waves sharing one workspace for large ones).
- *   HGX_OPTION_JOIN_TEAM waves that join one parent state: 1, 4 or 8 for every state, 0 automatic
- *                       (chosen the same way; binary states by bit sets, 16 lanes each, or by lists,
- *                       8 or 16 waves each).
+ *                       child, all by the general kernel (with 1, HGX_OPTION_EXPAND_LANES or the
+ *                       tuned lanes may split the wave); 0 automatic (default: children of one arity
+ *                       by size, down to 8 lanes each and up to 16 waves; others one wave for children
+ *                       whose workspace is small, a workgroup of 4 or 8 waves sharing one workspace
+ *                       for large ones).
+ *   HGX_OPTION_JOIN_TEAM waves that join one parent state: 1, 4 or 8 for every state, all by the
+ *                       general kernel; 0 automatic (chosen the same way; binary states by bit sets,
+ *                       16 lanes each, or by lists, 8 or 16 waves each).
  *   HGX_OPTION_EXPAND_LANES lanes that rewrite and hash one child when one wave is the team:
  *                       64, or 32 / 16 (sub-wave teams: two or four children per wave, each in
  *                       its own workspace), for every size class whose wave workspaces fit a
