@@ -27,14 +27,14 @@ struct LargeSizes {
         z.NN = (ne ? ne : 1) * A * (A - 1);
         z.CAP = z.NL + z.NL / 2 + 8;             // set slots: load factor 0.67 at most, and 0.83 where
         if (8u * z.NL + 4u * z.CAP > 140000u) z.CAP = z.NL + z.NL / 5 + 8;   // the LDS is nearly filled
-        if (z.CAP < z.NN / 2 + 1) z.CAP = z.NN / 2 + 1;      // the order of one list of every entry
+        if (z.CAP < z.NN / 2 + 1) z.CAP = z.NN / 2 + 1;      // the sorted lists, if all are long
         z.NLONG = z.NN / 9 + 1;
         z.NHUGE = z.NN / 65 + 1;
         return z;
     }
     // LDS held whatever the layout, and the rest
     __host__ __device__ uint32_t hot() const {
-        return 8 * NL + 8 * NHUGE + ((4 * CAP + 7u) & ~7u) + ((2 * NHUGE + 7u) & ~7u) + 256;
+        return 8 * NL + ((4 * CAP + 7u) & ~7u) + ((2 * NHUGE + 7u) & ~7u) + 256;
     }
     __host__ __device__ uint32_t rest() const {
         auto al = [](uint32_t b) { return (b + 7u) & ~7u; };
@@ -44,8 +44,7 @@ struct LargeSizes {
 
 struct LargeSpace {
     uint64_t* cur;      // [NL] LDS: occurrences per position (16 bits each), then colours
-    uint64_t* hres;     // [NHUGE] LDS: colours of the vertices with lists above 64 entries
-    uint32_t* set;      // [CAP] LDS: cursors; distinct-count set (label + 1); a list's order; components
+    uint32_t* set;      // [CAP] LDS: cursors; distinct-count set (label + 1); sorted lists; components
     uint32_t* word;     // [4] LDS
     uint16_t* hl;       // [NHUGE] LDS: vertices with lists above 64 entries
     uint64_t* red;      // [16] LDS: the team's reductions
@@ -61,7 +60,6 @@ struct LargeSpace {
 template <bool ALL>
 __device__ __forceinline__ void large_bind(LargeSpace& s, uint8_t* lds, uint8_t* mem, const LargeSizes& z) {
     s.cur = (uint64_t*)carve(lds, 8 * z.NL);
-    s.hres = (uint64_t*)carve(lds, 8 * z.NHUGE);
     s.set = (uint32_t*)carve(lds, 4 * z.CAP);
     s.word = (uint32_t*)carve(lds, 16);
     s.hl = (uint16_t*)carve(lds, 2 * z.NHUGE);
@@ -117,6 +115,40 @@ __device__ __forceinline__ uint32_t row_rank_from(uint64_t x, uint32_t i) {
     }
 }
 __device__ __forceinline__ uint32_t row_rank(uint64_t x, uint32_t i) { return row_rank_from<1>(x, i); }
+
+// Entries [a0, a0 + 64) of the list [b, b + n) to their places in order, by a wave: every entry's value comes
+// by in turn, 64 at a time by lane reads (equal ones by place).
+__device__ __forceinline__ void large_rank_unit(const LargeSpace& s, uint16_t* order, uint32_t b, uint32_t n,
+                                                uint32_t a0, uint32_t lane) {
+    auto entry = [&](uint32_t j) { return (uint32_t)s.nb[b + (j < n ? j : 0u)]; };
+    const uint32_t tx = entry(a0 + lane);
+    const uint64_t x = fnv(s.cur[tx >> 2], tx & 3u);
+    uint32_t r = 0;
+    uint32_t ty = entry(lane);
+    for (uint32_t c0 = 0; c0 < n; c0 += WAVE) {
+        const uint64_t y = fnv(s.cur[ty >> 2], ty & 3u);
+        ty = entry(c0 + WAVE + lane);                         // (the next ones' read meanwhile)
+        const uint32_t m = n - c0 < WAVE ? n - c0 : WAVE;
+        auto at = [&](uint32_t i) {
+            return ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(y >> 32), (int)i) << 32) |
+                   (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)y, (int)i);
+        };
+        if (c0 < a0) {
+#pragma unroll 8
+            for (uint32_t i = 0; i < m; ++i) r += at(i) <= x ? 1u : 0u;
+        } else if (c0 > a0) {
+#pragma unroll 8
+            for (uint32_t i = 0; i < m; ++i) r += at(i) < x ? 1u : 0u;
+        } else {
+#pragma unroll 8
+            for (uint32_t i = 0; i < m; ++i) {
+                const uint64_t z = at(i);
+                r += (z < x || (z == x && i < lane)) ? 1u : 0u;
+            }
+        }
+    }
+    if (a0 + lane < n) order[b + r] = (uint16_t)tx;
+}
 
 // ev: the state's edges at stride A in global memory; every edge has arity ua (UA when it is known).
 template <uint32_t UA, bool ALL, class TM>
@@ -199,47 +231,37 @@ __device__ __forceinline__ uint64_t wl_hash_large(LargeSpace s, const TM& tm, co
     const uint32_t w = l / WAVE, lane = lane_id();
     for (uint32_t it = 0; it < WL_MAX_ITERS; ++it) {
         tm.sync();
-        // Lists above 64 entries, one after another by the workgroup, through the next colours' memory
-        // (values recomputed for a list that does not fit it).
+        // Lists above 64 entries: 64 of a list's entries against all of it is a wave's unit of work, dealt
+        // to the waves in turn over all lists, the entries left in order in LDS; then a lane folds a list.
+        // (One list after another by the workgroup, folded from global memory: 2,000 edges on 40 vertices
+        // 1.96 ms, 0.14 so, 0.22 by the general hash; 12,000 on 200 0.56, general 3.0.)
         uint16_t* order = (uint16_t*)s.set;
-        for (uint32_t k = 0; k < nhuge; ++k) {
-            const uint32_t b = s.off[s.hl[k]], n = s.off[s.hl[k] + 1] - b;
-            const bool stored = n <= s.NL;
-            auto value = [&](uint32_t j) {
-                const uint32_t t = s.nb[b + j];
-                return fnv(s.cur[t >> 2], t & 3u);
-            };
-            if (stored) {
-                for (uint32_t j = l; j < n; j += N) s.nxt[j] = value(j);
-                tm.sync();
+        uint32_t u = (uint32_t)__builtin_amdgcn_readfirstlane((int)w);
+        for (uint32_t k0 = 0; k0 < nhuge; k0 += WAVE) {
+            const uint32_t hv = k0 + lane < nhuge ? s.hl[k0 + lane] : s.hl[0];
+            const uint32_t hb = s.off[hv], hn = s.off[hv + 1] - hb;
+            const uint32_t m = nhuge - k0 < WAVE ? nhuge - k0 : WAVE;
+            for (uint32_t k = 0; k < m; ++k) {
+                const uint32_t b = (uint32_t)__builtin_amdgcn_readlane((int)hb, (int)k);
+                const uint32_t n = (uint32_t)__builtin_amdgcn_readlane((int)hn, (int)k);
+                const uint32_t units = (n + WAVE - 1) / WAVE;
+                for (; u < units; u += N / WAVE) large_rank_unit(s, order, b, n, u * WAVE, lane);
+                u -= units;
             }
-            for (uint32_t j = l; j < n; j += N) {
-                const uint64_t x = value(j);
-                uint32_t r = 0;
-                if (stored) {
-#pragma unroll 8
-                    for (uint32_t i = 0; i < n; ++i) {
-                        const uint64_t y = s.nxt[i];
-                        r += (y < x || (y == x && i < j)) ? 1u : 0u;
-                    }
-                } else {
-                    for (uint32_t i = 0; i < n; ++i) {
-                        const uint64_t y = value(i);
-                        r += (y < x || (y == x && i < j)) ? 1u : 0u;
-                    }
-                }
-                order[r] = (uint16_t)j;
-            }
-            tm.sync();
-            if (l == 0) {
-                uint64_t h = s.cur[s.hl[k]];
-#pragma unroll 8
-                for (uint32_t i = 0; i < n; ++i) h = fnv(h, stored ? s.nxt[order[i]] : value(order[i]));
-                s.hres[k] = h;
-            }
-            tm.sync();
         }
-        for (uint32_t k = l; k < nhuge; k += N) s.nxt[s.hl[k]] = s.hres[k];
+        if (nhuge) {
+            tm.sync();
+            for (uint32_t k = l; k < nhuge; k += N) {
+                const uint32_t v = s.hl[k], b = s.off[v], e = s.off[v + 1];
+                uint64_t h = s.cur[v];
+#pragma unroll 8
+                for (uint32_t i = b; i < e; ++i) {
+                    const uint32_t t = order[i];
+                    h = fnv(h, fnv(s.cur[t >> 2], t & 3u));
+                }
+                s.nxt[v] = h;
+            }
+        }
         // 9 to 16 entries: four lists a wave, an entry per lane of a row, ranked against the row's
         // others by rotation and folded by shifting them down to its first lane
         for (uint32_t k0 = 4 * w; k0 < nmed; k0 += 4 * (N / WAVE)) {

@@ -1,6 +1,6 @@
 """GPU: dense states, most of whose neighbour lists are long, against the oracle. Small children: more long
 entries than are numbered at once (several batches), lists on both sides of half of them, teams of one wave
-with different numbers of batches."""
+with different numbers of batches. Large states: lists around 64 entries and multiples, one list and hundreds."""
 import random
 
 import pytest
@@ -81,6 +81,47 @@ def test_small_dense_children_take_no_longer_than_by_the_general_kernel(ctx):
         own = _ms(ctx, "k_expand", batch)
         try:
             ctx.set_expand_team(1)
+            general = _ms(ctx, "k_expand", batch)
+        finally:
+            ctx.set_expand_team(0)
+        print(own, general)
+        assert own < general
+LARGE = [_dense(m, n, 2) for m, n in ((300, 2), (300, 9), (1200, 9), (2000, 25), (2000, 62), (4000, 64), (12000, 100),
+                                      (12000, 200))]
+LARGE += [_hubs(d, m, n) for d, m, n in (([63, 64, 65, 66, 127, 128, 129, 130], 300, 100), ([1000, 65], 900, 9),
+                                         ([70] * 70, 400, 300), ([64, 4000], 300, 40))]
+LARGE += [_dense(900, 20, 3), _dense(900, 40, 3), _dense(700, 10, 4), _dense(700, 60, 4)]
+
+
+def _compact(edges):
+    ids = {}
+    return [[ids.setdefault(v, len(ids)) for v in e] for e in edges]
+
+
+@pytest.mark.parametrize("i", range(len(LARGE)))
+def test_large_dense_states_equal_oracle(ctx, i):
+    state = _compact(LARGE[i])
+    other = state[:]
+    random.Random(i).shuffle(other)
+    got = ctx.wl_hash([state, other])
+    assert [int(x) for x in got] == [po.wl_hash(state)] * 2
+    a = len(state[0])
+    top = max(v for e in state for v in e)
+    req = Request([rule_from_lists([[0] * a], [[0] * a, list(range(a))])],
+                  state + [[top + 1 + k] * a for k in range(3)], 1, flags=REL)
+    assert_exact(ctx.evolve(req), po.evolve(req), tr=True)
+
+
+def test_large_dense_children_take_no_longer_than_by_the_general_kernel(ctx):
+    """0.6 and 0.2 of it; with one list above 64 entries after another the first took 9 times as long."""
+    for m, n in ((2000, 40), (12000, 200)):
+        state = _dense(m, n, 2)
+        req = Request([rule_from_lists([[0, 0]], [[0, 0], [0, 1]])], state + [[n + k] * 2 for k in range(3)], 1, flags=0x1)
+        batch = ctx.prepare([req])
+        ctx.evolve_batch(batch)
+        own = _ms(ctx, "k_expand", batch)
+        try:
+            ctx.set_expand_team(8)
             general = _ms(ctx, "k_expand", batch)
         finally:
             ctx.set_expand_team(0)
