@@ -568,6 +568,8 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
                     jcls[i] = k;
                 }
             }
+            // binary states by the kernels of their own, unless the general one is asked for
+            const bool own_join = !ctx_->join_team && !ctx_->general_only;
             // One launch per size class, each with LDS staging sized for its class; states outside
             // the launches (requests not advancing) keep the zero count set here.
             auto launch_classes = [&](bool emit, std::vector<ExpandClass>& cls, const char* name,
@@ -609,7 +611,7 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
                     // lanes per state (batched count pass 0.85 ms, 1.04 with 32; few states time
                     // alike), up to 32 workgroups per CU (0.94 ms at 8, 0.86 at 16).
                     const uint32_t nw = match_bits_words(mc.max_ne);
-                    if (x.uniform && nw && mc.max_nextv <= kMatchBitsLabels && !mc.fwd_n && !ctx_->join_team) {
+                    if (x.uniform && nw && mc.max_nextv <= kMatchBitsLabels && !mc.fwd_n && own_join) {
                         mc.lds_per_wave = match_bits_lds(mc.max_ne, mc.max_nextv, nw);
                         uint32_t lanes = ctx_->join_lanes ? ctx_->join_lanes : 16u;
                         while (lanes < 64 && (uint64_t)mc.lds_per_wave * (64 / lanes) > ctx_->max_lds) lanes *= 2;
@@ -626,7 +628,7 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
                     // served mix 2.24 -> 0.72 and 1.55 -> 0.53, one state of 12,001 edges, in global
                     // workspaces there, 1.43 -> 0.06 and 0.72 -> 0.11.
                     const uint32_t lists = match_lists_lds(mc.max_ne, mc.max_nextv);
-                    if (x.uniform && ctx_->forward != 1 && !ctx_->join_team && lists <= ctx_->max_lds) {
+                    if (x.uniform && ctx_->forward != 1 && own_join && lists <= ctx_->max_lds) {
                         mc.fwd_n = 0; mc.dmax = 0;
                         mc.lds_per_wave = lists;
                         const uint32_t tw = mc.max_ne <= 2048 && x.n >= ctx_->num_cu ? 8u : 16u;
@@ -972,6 +974,7 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
                 x.rpre.push_back((uint32_t)x.n);
             }
             put_ranges(cls, M);
+            const bool own_expand = !ctx_->expand_team && !ctx_->general_only;
             const uint64_t bytes = M * (8ull + 2ull * K) + parent_edges * (4ull * F_->v.A + 2) +
                                    EC * (4ull * A + 2) + M * 8ull;
             for (int k = 0; k < kExpandClasses; ++k) {
@@ -991,7 +994,7 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
                 // (a request of arity 5 and up in another class widens the generation's edges past
                 // both one-arity kernels)
                 if (ea.lean && A <= 4 && ea.max_child_ne <= kSmallMaxEdges && ea.max_nextv <= kSmallMaxLabels &&
-                    !ctx_->expand_team) {
+                    own_expand) {
                     const SmallShape sh = small_shape(ea, K, ctx_->expand_lanes, ctx_->max_lds, A);
                     ea.lds_per_wave = sh.lds;
                     timed(ctx_, st, "k_expand", (uint64_t)((double)bytes * x.n / M), x.n,
@@ -1000,7 +1003,7 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
                 }
                 // larger children of one arity whose colours fit the LDS: 360 children of 12,001
                 // edges 8.96 -> 0.89 ms, 20 k of 256 to 2,048 edges 4.7 -> 2.7
-                if (ea.lean && A <= 4 && !ctx_->expand_team && large_fits(ea.max_child_ne, ea.max_nextv, A) &&
+                if (ea.lean && A <= 4 && own_expand && large_fits(ea.max_child_ne, ea.max_nextv, A) &&
                     large_lds(ea.max_child_ne, ea.max_nextv, A, false) <= ctx_->max_lds) {
                     const LargeShape sh = large_shape(ea.max_child_ne, ea.max_nextv, A, ea.n_items, ctx_->max_lds,
                                                       ctx_->num_cu);

@@ -319,6 +319,8 @@ struct hgx_ctx {
     uint64_t flush_bytes = 0;                    // HGX_OPTION_COUNTER_FLUSH
     void* flush_buf = nullptr;                   // its buffer (hipMalloc'd, freed with the context)
     hgx::Tune tune;                              // launch shapes per size class
+    bool general_only = false;                   // hgx_autotune: the kernels whose shapes are tuned, for
+                                                 // every child and state
 };
 
 namespace hgx {

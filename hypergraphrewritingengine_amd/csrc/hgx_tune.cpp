@@ -6,12 +6,15 @@
 // waves per state, the lanes per state when one wave is the team (16 / 32 / 64), and the
 // workgroups per CU. Each candidate is run over a caller's prepared batch with the
 // launches event-timed per class, and each class keeps the fastest candidate (classes are separate
-// launches, so one sweep serves them all). Children of one arity and binary states take kernels whose
-// shapes follow from their sizes; the tuned shapes are those of the general kernels. The choice is kept in the context and written to a JSON
-// cache keyed by "<arch>:<CUs>", which hgx_ctx_create loads for its device (from HGX_TUNE_CACHE,
-// else tune_cache.json beside the library). None of the shapes changes a result -- the tests run
-// every lane count and team size against the oracle. The join order is not tuned: event numbering
-// follows the reference's join order (hypergraph/src/pattern.cpp:43-75), which fixes it.
+// launches, so one sweep serves them all). The shapes are those of the general kernels; children of
+// one arity and binary states take kernels of their own, whose shapes follow from their sizes, so the
+// sweep sends every child and state of the batch through the general ones (as such batches run
+// otherwise, candidates differ by noise alone). A class that the batch does not reach keeps its
+// shape. The choice is kept in the context and written to a JSON cache keyed by "<arch>:<CUs>", which
+// hgx_ctx_create loads for its device (from HGX_TUNE_CACHE, else tune_cache.json beside the library).
+// None of the shapes changes a result -- the tests run every lane count and team size against the
+// oracle. The join order is not tuned: event numbering follows the reference's join order
+// (hypergraph/src/pattern.cpp:43-75), which fixes it.
 #include <hip/hip_runtime.h>
 
 #include <dlfcn.h>
@@ -143,6 +146,11 @@ extern "C" int hgx_autotune(hgx_ctx* ctx, const hgx_batch* batch, uint32_t reps,
         // forced options would hide what the candidates change
         const uint32_t saved_lanes = ctx->expand_lanes, saved_jt = ctx->join_team, saved_et = ctx->expand_team,
                        saved_jl = ctx->join_lanes;
+        struct GeneralOnly {                                   // until the tuner returns or throws
+            hgx_ctx* c;
+            explicit GeneralOnly(hgx_ctx* x) : c(x) { c->general_only = true; }
+            ~GeneralOnly() { c->general_only = false; }
+        } general(ctx);
         const bool saved_on = ctx->prof.on, saved_cls = ctx->prof.by_class;
         const Tune saved = ctx->tune;
         ctx->expand_lanes = 0; ctx->join_team = 0; ctx->expand_team = 0; ctx->join_lanes = 0;
