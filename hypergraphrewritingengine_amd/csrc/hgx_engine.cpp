@@ -542,8 +542,6 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
             ma.pm_moff = prev_.moff;
             ma.KL = KL;
             ma.small = small ? 1u : 0u;
-            // small rules: the count pass keeps each seed's match count for the emit pass
-            ma.seedcnt = small ? dalloc<uint16_t>(tmp, 2 * std::max<uint64_t>(1, F_->n_edges)) : nullptr;
             ma.dmax = fwd ? std::min(ctx_->delta_cap, 16384u / (2u * KL + 8u)) : 0u;   // <= 16 KiB LDS
             ma.budget = d_budget_;
             ma.run_acc = (unsigned long long*)d_run_acc_;
@@ -649,6 +647,10 @@ uint32_t Engine::step_impl(std::vector<std::shared_ptr<RunRec>>& admitted) {
                         gws_grid = launch_grid((uint32_t)x.n, 1, cap);
                         mc.scratch = (uint8_t*)tmp.alloc((size_t)gws_grid * mc.lds_per_wave);
                     }
+                    // small rules: this kernel's count pass keeps each seed's match count for its emit pass
+                    if (!emit && small && !ma.seedcnt)
+                        ma.seedcnt = dalloc<uint16_t>(tmp, 2 * std::max<uint64_t>(1, F_->n_edges));
+                    mc.seedcnt = ma.seedcnt;
                     // sub-wave teams for small states, when the wave's workspaces fit a workgroup
                     uint32_t lanes = 64;
                     if (team == 1 && !mc.scratch) {

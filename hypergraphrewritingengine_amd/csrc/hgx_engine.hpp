@@ -202,10 +202,10 @@ private:
     // memory, flush() moves all of them in one launch (k_move), settle() flushes, waits for the
     // stream and hands out what get() asked for. A copy by itself costs the runtime's staging and
     // a launch of its own: a generation took 10 to 20 of them, 5 us each. Every put() is flushed
-    // before the launch that reads it. The staging is a lease of the context's pinned buffers, free
-    // again once the stream is idle (each step ends so); under capture it is the engine's own and
-    // lives as long, since a replay reads it again. Larger transfers, and those past the staging,
-    // are copies of their own.
+    // before the launch that reads it. The staging is a lease of the context's pinned buffers that the
+    // engine holds; its bytes are free again once the stream is idle (each step ends so). Under capture
+    // it is the engine's own and lives as long, since a replay reads it again. Larger transfers, and
+    // those past the staging, are copies of their own.
     static constexpr size_t kMoveMax = (size_t)256 << 10;
     void put(void* dst, const void* src, size_t bytes, hipStream_t st);
     void get(void* dst, const void* src, size_t bytes, hipStream_t st);

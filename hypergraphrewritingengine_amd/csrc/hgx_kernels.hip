@@ -1468,8 +1468,8 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W, W == 1 ? 4 : 1) void k_expan
     }
 }
 
-// k_expand for small children of one arity (ExpandArgs::small): the same records, with the hash of
-// hgx_wl_small.hpp. Labels are bytes, so the rewrite leaves its edges in LDS as the hash reads them;
+// k_expand for small children of one arity (at most kSmallMaxEdges edges and kSmallMaxLabels labels, a stride of
+// at most 4): the same child, with the hash of hgx_wl_small.hpp. Labels are bytes, so the rewrite leaves its edges in LDS as the hash reads them;
 // a kept edge's place is its position less the consumed positions below it (two words of bits), so
 // the copy needs no compaction and its loads do not wait for each other.
 template <uint32_t UA, uint32_t G>

@@ -190,7 +190,7 @@ uint32_t match_bits_lds(uint32_t max_ne, uint32_t max_nextv, uint32_t nw);
 hipError_t launch_match_bits(const MatchArgs& a, bool emit, uint32_t grid_cap, uint32_t wpb, hipStream_t st,
                              uint32_t lanes);
 // Larger binary states (the same conditions, up to 65,535 edges and labels): LDS per workgroup, and the
-// launch with 4, 8 or 16 waves per state.
+// launch with 8 or 16 waves per state.
 uint32_t match_lists_lds(uint32_t max_ne, uint32_t max_nextv);
 hipError_t launch_match_lists(const MatchArgs& a, bool emit, uint32_t grid, uint32_t team, hipStream_t st);
 uint32_t expand_lds_per_wave(uint32_t max_child_ne, uint32_t max_nv, uint32_t max_nextv, uint32_t A, bool lean);
